@@ -33,13 +33,14 @@ PER_FILE = {
     "qk_prepass.hip": ["-ffp-contract=off"],
     "rot_q8.hip": ["-ffp-contract=off"],
     "gemm.hip": ["-ffp-contract=off"],
+    "gemm_ksplit.hip": ["-ffp-contract=off"],
     # score MFMAs with VGPR results (the softmax reads them), P V accumulators in AGPRs (inline assembly)
     "attention_wave.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 # sources whose inline assembly (MFMAs, DPP fmacs) is checked for hazards in the generated code (isa_check.py)
 ISA_CHECKED = ["attention_wave.hip", "qk_prepass.hip", "rot_q8.hip"]
 SOURCES = ["attention_wave.hip", "attention.hip", "capi.hip", "qk_prepass.hip", "rot_q8.hip",
-           "gemm.hip"]
+           "gemm.hip", "gemm_ksplit.hip"]
 
 
 def hipcc() -> str:

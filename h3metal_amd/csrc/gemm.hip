@@ -21,42 +21,13 @@
 // outputs half a tile at a time) and leaves as 16-byte row stores. The residual form keeps C in the
 // accumulators (a lane holds one column) and reads X, writes X per wave without barriers, 128 contiguous bytes
 // of two rows per access, so one wave's epilogue overlaps the other waves' MFMAs.
-#include "h3hip_internal.h"
+#include "gemm_common.h"
 
 #include <algorithm>
 #include <cstring>
-#include <type_traits>
 
 namespace h3 {
 namespace {
-
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-// operand types of a kernel: int8 (q8), half (f16, and h8 after its weights are widened), bfloat (bf16)
-enum { A_I8 = 0, A_F16 = 1, A_BF16 = 2 };
-// epilogue scaling: sa[m] * sw[n] (q8), sw[n] (h8), none (f16, bf16)
-enum { S_ROW_COL = 0, S_COL = 1, S_NONE = 2 };
-
-enum { T_BF16 = 1, T_F16 = 2, T_F32 = 3 };
-
-template <int AT>
-using AccOf = typename std::conditional<AT == A_I8, i32x16, f32x16>::type;
-
-// one 32 x 32 product over a 32-byte K slice per lane half (32 int8 or 16 16-bit values of K)
-template <int AT>
-__device__ __forceinline__ AccOf<AT> mma(i32x4 a, i32x4 b, AccOf<AT> c) {
-  if constexpr (AT == A_I8) return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
-  else if constexpr (AT == A_F16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
-                                                  0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                   0, 0, 0);
-}
 
 constexpr int KS = 64;                           // K bytes per step
 constexpr int NWG = 8;                           // waves per workgroup
@@ -83,7 +54,6 @@ using TileSmall = GTile<128, 128>;
 
 // 16-byte piece p of LDS row r (64 bytes) sits at slot p ^ ((r / 4) % 4)
 __device__ __forceinline__ int swz(int row, int piece) { return row * KS + ((piece ^ ((row >> 2) & 3)) << 4); }
-
 
 template <int OT>
 __device__ __forceinline__ void store_out(char *p, float v) {
@@ -391,6 +361,53 @@ __global__ __launch_bounds__(256) void widen_i8_f16(const signed char *__restric
   *(f16x8 *)(out + n * K + k) = h;
 }
 
+// How a product runs: which tiles, and for the 256 x 256 ones how many rows its main launch takes (the trailing rows
+// then run as 128 x 128 tiles).
+struct Plan {
+  int ksplit = -1;       // a configuration of gemm_ksplit.hip, or -1
+  bool small = false;    // 128 x 128 tiles throughout
+  int main_rows = 0;     // rows of the 256 x 256 tiles
+};
+
+// The plan of least estimated time. A configuration takes rounds (tiles over CUs, rounded up) times a cost per tile
+// that is linear in the bytes of a row of A's K: us = fixed + per_kb * K bytes / 1024, fitted to a sweep of 3 formats
+// x 11 row counts (16 to 3300) x 5 (N, K) pairs (N 1024 to 12288, K 1024 to 10240) on an MI355X; the plan's time was
+// within 1% of the best configuration's on average over the sweep, 1.31x of it at worst, and never above that of
+// the 256 x 256 tiles with their tail launch (which it beat 2.8x on average). 256 x 256 tiles: when the last round of tiles would leave more than
+// half the CUs idle, its rows may go to a second launch of 128 x 128 tiles (0.45 of a big tile's time each).
+// h8 outside gemm_ksplit.hip also widens its weights first (about 14 us for 4096 x 4096).
+Plan make_plan(const GemmParams &p, int wfmt, int es, bool can_ksplit) {
+  Plan pl;
+  pl.main_rows = p.M;
+  const int cus = cu_count();
+  if (cus <= 0) return pl;
+  const double kb = (double)p.K * es / 1024, widen = wfmt == 6 ? 3 + 0.7e-6 * (double)p.N * p.K : 0;
+  auto tiles = [&](long rows, int tm, int tn) { return ((rows + tm - 1) / tm) * (((long)p.N + tn - 1) / tn); };
+  auto rounds = [&](long n) { return (double)((n + cus - 1) / cus); };
+  constexpr int BT = TileBig::TM, ST = TileSmall::TM;
+  const long ntm = (p.M + BT - 1) / BT, ntn = (p.N + BT - 1) / BT, nt = ntm * ntn, R = nt % cus;
+  double r = rounds(nt);
+  const long tr = (R + ntn - 1) / ntn;  // trailing rows of tiles that hold the last round's tiles
+  if (R > 0 && 2 * R <= cus && tr < ntm) {
+    const long mrows = (ntm - tr) * BT;
+    const double t = rounds((ntm - tr) * ntn) + 0.45 * rounds(tiles(p.M - mrows, ST, ST));
+    if (t < r) r = t, pl.main_rows = (int)mrows;
+  }
+  // the smaller tiles have to be estimated 12% faster: near the line the estimate's error decides, and the residual
+  // form, whose end costs more on small tiles, lost 7% there
+  double best = 0.88 * (widen + r * (9.5 + 9.5 * kb));
+  const double small = widen + rounds(tiles(p.M, ST, ST)) * (4.0 + 3.7 * kb);
+  if (small < best) best = small, pl.small = true;
+  if (!can_ksplit) return pl;
+  static const struct { int tm, tn; double fixed, per_kb; } ks[] = {
+      {32, 32, 1.7, 0.82}, {64, 64, 4.1, 1.42}, {96, 64, 5.6, 1.75}, {96, 128, 9.2, 2.45}};  // by KSPLIT_*
+  for (int k = 0; k < (wfmt == 1 ? 3 : 4); k++) {
+    const double t = rounds(tiles(p.M, ks[k].tm, ks[k].tn)) * (ks[k].fixed + ks[k].per_kb * kb);
+    if (t < best) best = t, pl.ksplit = k;
+  }
+  return pl;
+}
+
 // Formats: WFMT 1 (q8: int8 A and W, sa[m] sw[n]), 4 (f16: half A and W), 5 (bf16), 6 (h8: half A, int8 W with
 // sw[n]; W widened to half first).
 template <int OT, int EPI, bool HAS_BIAS, int WFMT>
@@ -454,20 +471,12 @@ int launch_gemm(const Pipeline &pl, const Exec &ex, const Arg *a, int nargs, con
       *err = std::string(i ? "w" : "a") + " must be 16-byte aligned";
       return -1;
     }
-  const void *wptr = a[1].ptr;
-  if constexpr (WFMT == 6) {
-    // the widened weights go to the stream's scratch buffer; the product reads them with a dense row stride
-    const size_t wbytes = (size_t)N * p.K * 2;
-    if (wbytes > ex.ws_bytes) {
-      *err = "the widened h8 weights need " + std::to_string(wbytes) + " bytes of scratch, " +
-             std::to_string(ex.ws_bytes) + " are reserved (h3_reserve_workspace)";
-      return -1;
-    }
-    _Float16 *wh = (_Float16 *)ex.ws;
-    hipLaunchKernelGGL(widen_i8_f16, dim3((unsigned)((p.K / 8 + 255) / 256), (unsigned)N), dim3(256), 0, ex.stream,
-                       (const signed char *)a[1].ptr, wh, p.N, p.K, p.w_stride);
-    wptr = wh;
-    p.w_stride = p.K;
+  if (WFMT == 6 && N * p.K * 2 > ex.ws_bytes) {
+    // the widened weights of the large-tile path; checked for every call, so that what is accepted does not depend
+    // on the tile that a shape gets
+    *err = "the widened h8 weights need " + std::to_string(N * p.K * 2) + " bytes of scratch, " +
+           std::to_string(ex.ws_bytes) + " are reserved (h3_reserve_workspace)";
+    return -1;
   }
   // 16-byte vector access to the output (and the column vectors) when alignment and N allow it
   constexpr int VE = 16 / OSZ;
@@ -475,10 +484,30 @@ int launch_gemm(const Pipeline &pl, const Exec &ex, const Arg *a, int nargs, con
   const bool vec = al16(a[4].ptr) && (p.c_stride * OSZ) % 16 == 0 && p.N % VE == 0 &&
                    (SM == S_NONE || al16(a[2].ptr)) && (!HAS_BIAS || al16(a[5].ptr)) &&
                    (!EPI || (al16(a[7].ptr) && p.g_stride % 4 == 0));
-  // One grid of 256 x 256 tiles; when its last round of tiles would leave more than half the CUs idle, the
-  // trailing rows of tiles go to a second launch of 128 x 128 tiles (the same kernel on the sub-problem of those
-  // rows: A, sa, rtype and the output offset by the first row), if that shortens the estimated time (a small
-  // tile taken as 0.45 of a big one's time).
+  const Plan plan = make_plan(p, WFMT, ES, WFMT != 6 || p.w_stride % 16 == 0);
+  if (plan.ksplit >= 0) {
+    const GemmArgs g{a[0].ptr,
+                     a[1].ptr,
+                     SM != S_NONE ? (const float *)a[2].ptr : nullptr,
+                     SM == S_ROW_COL ? (const float *)a[3].ptr : nullptr,
+                     a[4].ptr,
+                     HAS_BIAS ? (const float *)a[5].ptr : nullptr,
+                     EPI ? (const unsigned char *)a[6].ptr : nullptr,
+                     EPI ? (const float *)a[7].ptr : nullptr,
+                     ntypes,
+                     vec};
+    return launch_gemm_ksplit(WFMT, plan.ksplit, OT, EPI, g, p, ex.stream, err);
+  }
+  const void *wptr = a[1].ptr;
+  if constexpr (WFMT == 6) {
+    // the widened weights go to the stream's scratch buffer; the product reads them with a dense row stride
+    _Float16 *wh = (_Float16 *)ex.ws;
+    hipLaunchKernelGGL(widen_i8_f16, dim3((unsigned)((p.K / 8 + 255) / 256), (unsigned)N), dim3(256), 0, ex.stream,
+                       (const signed char *)a[1].ptr, wh, p.N, p.K, p.w_stride);
+    wptr = wh;
+    p.w_stride = p.K;
+  }
+  // The sub-problem of `rows` rows from row0 (A, sa, rtype and the output offset by the first row) on one tile size
   auto launch = [&](auto tl, int row0, int rows) -> int {
     using TL = decltype(tl);
     auto kern = gemm_kernel<OT, EPI, HAS_BIAS, AT, SM, TL>;
@@ -505,22 +534,9 @@ int launch_gemm(const Pipeline &pl, const Exec &ex, const Arg *a, int nargs, con
                        q, ntm, ntn, ntypes, vec);
     return 0;
   };
-  constexpr int BT = TileBig::TM, ST = TileSmall::TM;
-  const int ntm = (p.M + BT - 1) / BT, ntn = (p.N + TileBig::TN - 1) / TileBig::TN;
-  const int cus = cu_count();
-  int main_rows = p.M;
-  if (cus > 0) {
-    const long nt = (long)ntm * ntn, R = nt % cus;
-    const int tr = (int)((R + ntn - 1) / ntn);  // trailing rows of tiles that hold the last round's tiles
-    if (R > 0 && 2 * R <= cus && tr < ntm) {
-      const int mrows = (ntm - tr) * BT;
-      const long small = (long)((p.M - mrows + ST - 1) / ST) * ((p.N + ST - 1) / ST);
-      const double t_split = (double)(((long)(ntm - tr) * ntn + cus - 1) / cus) + 0.45 * ((small + cus - 1) / cus);
-      if (t_split < (double)((nt + cus - 1) / cus)) main_rows = mrows;
-    }
-  }
-  if (launch(TileBig{}, 0, main_rows)) return -1;
-  if (main_rows < p.M && launch(TileSmall{}, main_rows, p.M - main_rows)) return -1;
+  if (plan.small) return launch(TileSmall{}, 0, p.M);
+  if (launch(TileBig{}, 0, plan.main_rows)) return -1;
+  if (plan.main_rows < p.M && launch(TileSmall{}, plan.main_rows, p.M - plan.main_rows)) return -1;
   return 0;
 }
 

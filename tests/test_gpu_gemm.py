@@ -383,3 +383,39 @@ def test_float_format_refusals(gpu):
                  gate=gpu.upload(np.ones((1, 256), np.float32)), ksplit=2, tile=(1, 2, 4))
     with pytest.raises(GpuError):  # K must be a multiple of 32 for 16-bit operands
         ops.gemm(gpu, A, ops.QWeight("f16", wt.w, None, 256, 200, ws=256), out, 64, a_stride=256, tile=(1, 2, 4))
+
+
+@pytest.mark.parametrize("fmt", ["q8", "h8", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1, 36, 64), (33, 1000, 1088), (130, 4096, 1088), (97, 8192, 192),
+                                   (289, 4096, 1088), (385, 4100, 2112)])
+def test_few_tiles_bit_exact(gpu, fmt, M, N, K):
+    """Products of few output tiles (the waves of a workgroup split K): each small tile (32 x 32, 64 x 64, 96 x 64,
+    and for h8 at 385 rows 96 x 128) with ragged rows and columns, fewer K slices than waves and a last half slice.
+    The operands are small integers, so every format's sums are whole numbers below 2^24, exact in float32 in any
+    order, and both epilogues are compared bit for bit."""
+    rng = np.random.default_rng(M + N + K)
+    a = rng.integers(-8, 9, size=(M, K), dtype=np.int8)
+    q = rng.integers(-127, 128, size=(N, K), dtype=np.int8)
+    assert K * 8 * 127 < 2 ** 24
+    sa, sw = (rng.uniform(0.001, 0.01, size=n).astype(np.float32) for n in (M, N))
+    b = rng.standard_normal(N).astype(np.float32)
+    acc = og.int_product(a, q)
+    if fmt == "q8":
+        A, W, v = gpu.upload(a), gpu.upload(q), og.epilogue(acc, sa, sw, b)
+    elif fmt == "h8":
+        A, W, v = gpu.upload(a.astype(np.float16)), gpu.upload(q), acc.astype(np.float32) * sw + b
+    else:
+        A, W = (gpu.upload(to_bf16(t.astype(np.float32)), "bf16") for t in (a, q))
+        v = acc.astype(np.float32) + b
+    wt = ops.QWeight(fmt, W, gpu.upload(sw) if fmt != "bf16" else None, N, K, bias=gpu.upload(b))
+    out, x0 = gpu.empty((M, N), "f32"), rng.standard_normal((M, N)).astype(np.float32)
+    types = rng.integers(0, 3, size=M).astype(np.uint8)
+    gates = rng.standard_normal((3, N)).astype(np.float32)
+    X = gpu.upload(x0)
+    SA = gpu.upload(sa) if fmt == "q8" else None
+    print(f"[gemm few tiles] {fmt} M={M} N={N} K={K}", flush=True)
+    ops.gemm(gpu, A, wt, out, M, sa=SA, tile=(1, 2, 4))
+    ops.gemm(gpu, A, wt, X, M, sa=SA, epi=1, rtype=gpu.upload(types), gate=gpu.upload(gates), tile=(1, 2, 4))
+    gpu.wait()
+    assert np.array_equal(out.numpy().view(np.uint32), v.view(np.uint32))
+    assert np.array_equal(X.numpy().view(np.uint32), (x0 + gates[types] * v).view(np.uint32))
