@@ -39,7 +39,7 @@ PER_FILE = {
 }
 # sources whose inline assembly (MFMAs, DPP fmacs) is checked for hazards in the generated code (isa_check.py)
 ISA_CHECKED = ["attention_wave.hip", "qk_prepass.hip", "rot_q8.hip"]
-SOURCES = ["attention_wave.hip", "attention.hip", "capi.hip", "qk_prepass.hip", "rot_q8.hip",
+SOURCES = ["attention_wave.hip", "attention.hip", "attention_small.hip", "capi.hip", "qk_prepass.hip", "rot_q8.hip",
            "gemm.hip", "gemm_ksplit.hip"]
 
 

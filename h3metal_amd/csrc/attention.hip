@@ -47,7 +47,8 @@
 //  * The 1-D grid is remapped so that each XCD (own L2) runs a contiguous
 //    range of (head, query-block) tiles, which then share one head's K/V in L2.
 //  * D = 128 without a causal mask (the DiT path) runs on the wave-pipelined
-//    kernel of attention_wave.hip; this file's kernel serves every other case.
+//    kernel of attention_wave.hip; this file's kernel serves every other case;
+//    calls too short for 256-row tiles run on attention_small.hip (small_tiles).
 #include "attention_common.h"
 
 #include <algorithm>
@@ -504,6 +505,43 @@ size_t attention_workspace_max(int cus) { return (size_t)std::max(cus, 1) * 384 
 
 namespace {
 
+// Whether a call runs on the small tiles of attention_small.hip: 0 no, else the 32-row query tiles per workgroup (1 or
+// 2). Decided by the estimated time (us) of both, from a sweep on an MI355X (head counts 4 to 512, 64 to 5000 rows,
+// head dims 64, 96, 128, int8 and 16-bit scores, causal and not):
+//  small tiles: 5 + c us per 1000 (32-query, 32-key) blocks, c = 0.5, 0.7, 1.0 for head dim 64, 96, 128 (two query tiles
+//  per workgroup at head dim 96: 12 + 0.95 per 1000 (64, 32) blocks, less from about 50 000 blocks on);
+//  256-row tiles: a start plus a time per 64-key block of each round of workgroups, plus the merge of a split last
+//  round. With a causal mask the longest tile or the mean load of a CU.
+// Measured, 256-row -> small tiles: bf16 H 4 256 rows 15.7 -> 9.0, int8 H 32 600 rows 33.8 -> 19.5 (1300: 58.9 -> 53.1,
+// 1800: 70 against 90, not taken), causal H 32 512 rows 24.7 -> 11.2, head dim 96 H 16 1037 rows 33.3 -> 22.8 (3000: 78
+// against 82, not taken), head dim 64 H 128 256 rows 26.8 -> 9.8. The small tiles have to be estimated 7% faster.
+int small_tiles(int d, bool b16, bool causal, bool wave, size_t ws_bytes, const AttnParams &p) {
+  const long cus = cu_count();
+  if (cus <= 0 || (uint64_t)(p.L + 256) * d * 2 > 0x7fffffffull) return 0;  // its byte offsets must stay below 2^31
+  const long nq = (p.Lq + 31) / 32, nk = (p.L + 31) / 32;
+  if (nq * p.H > 0x7fffffffL / 256) return 0;
+  const long nqb = (p.Lq + 255) / 256, tiles = nqb * p.H, nb = (p.L + BK - 1) / BK;
+  double steps = (double)nq * nk * p.H, other;
+  if (causal) {
+    auto keys = [&](long rows) { return std::max(0L, std::min((long)p.L, rows + p.causal_off)); };
+    steps = 0;
+    for (long t = 0; t < nq; t++) steps += (double)((keys(32 * t + 32) + 31) / 32) * p.H;
+    double total = 0;
+    for (long t = 0; t < nqb; t++) total += (double)((keys(256 * t + 256) + BK - 1) / BK) * p.H;
+    other = 5 + 2.2 * std::max((double)((keys(256 * nqb) + BK - 1) / BK), total / cus);
+  } else {
+    const double start = wave ? (b16 ? 12 : 15) : 5, per = wave ? (b16 ? 1.55 : 1.8) : d == 128 ? 2.2 : 1.65;
+    const long R = tiles % cus;
+    const size_t fit = R ? ws_bytes / ((size_t)256 * (d + 4) * sizeof(float) * R) : 0;
+    const long s = R ? std::min(std::min(cus / R, nb / 2), (long)fit) : 0;
+    const double last = R == 0 ? 0 : s >= 2 ? (double)((nb + s - 1) / s) + (wave ? 7 : 16) / per : (double)nb;
+    other = start + per * ((double)(tiles / cus) * nb + last);
+  }
+  const double one = 5 + (d == 64 ? 0.5e-3 : d == 96 ? 0.7e-3 : 1.0e-3) * steps;
+  const double two = d == 96 ? 12 + 0.95e-3 * steps / 2 : 2 * one;
+  return std::min(one, two) < 0.93 * other ? (two < one ? 2 : 1) : 0;
+}
+
 // Host side: validation (every access the kernel makes must fall inside the
 // bound buffers) and launch.
 template <int D, int QKT, int VT, int OT, bool CAUSAL, bool DUMP>
@@ -597,6 +635,10 @@ int launch_attention(const Pipeline &pl, const Exec &ex, const Arg *args, int na
     return -1;
   }
   if (p.Lq == 0) return 0;
+  if (!DUMP || usew) {
+    const int nu = pl.ival[1] ? small_tiles(D, QKT != T_I8, CAUSAL, usew, ex.ws_bytes, p) : 0;
+    if (nu) return launch_attention_small(D, QKT, VT, OT, nu, CAUSAL, DUMP, ex, args, p, err);
+  }
   const int BQ = usew ? WAVE_BQ : C::BQ;
   const int nqb = (p.Lq + BQ - 1) / BQ;
   const long ntiles = (long)nqb * p.H;
@@ -689,9 +731,11 @@ int type_of(const std::string &s) {
 // reference's tuning macros WM, BK, KPAD, DB, PVORDER, VX, SLACK are accepted
 // as integers and do not change the gfx950 kernel (its tiles are its own).
 // SPLIT (this build's, default 1): allow the tail split of a partly filled
-// last round of workgroups; SPLIT=0 runs every tile whole. GROUPS (this
-// build's) 0 or 1: the wave-pipelined kernel for HD 128 without a causal mask
-// (the values that selected other kernels for it are refused).
+// last round of workgroups, and the small tiles whose waves split the keys;
+// SPLIT=0 runs every tile whole. GROUPS (this build's): 1 the wave-pipelined
+// kernel for HD 128 without a causal mask at every size, 0 (the default) the
+// small tiles where they are faster (the values that selected other kernels are
+// refused).
 bool make_attention(const std::string &fn, const Macros &m, Pipeline *pl, std::string *err) {
   const bool dump = fn == "attention_scores";
   if (fn != "attention" && !dump) {
@@ -742,6 +786,7 @@ bool make_attention(const std::string &fn, const Macros &m, Pipeline *pl, std::s
   const int ksel = hd == 128 && !causal ? 1 : 0;
   pl->threads = ksel == 1 ? WAVE_THREADS : NW * 64;
   pl->ival[0] = split != 0;
+  pl->ival[1] = split != 0 && groups == 0;  // the small tiles split the keys, and GROUPS=1 names a kernel
   pl->ival[2] = ksel;
   return true;
 }

@@ -37,6 +37,12 @@ constexpr int WAVE_THREADS = 256;       // its workgroup: 4 waves, one per SIMD
 int launch_attention_wave(int qkt, int vt, int ot, bool dump, const Exec &ex, const Arg *args, const AttnParams &p,
                           int nqb, const Split &sp, std::string *err);
 
+// The kernel of few and short tiles (attention_small.hip): any head dim, with or without a causal mask, 32 nu query
+// rows per workgroup (nu 1, or 2 at head dim 96); `dump` as below (head dim 128). Byte offsets of a head's K and V rows
+// must stay below 2^31.
+int launch_attention_small(int d, int qkt, int vt, int ot, int nu, bool causal, bool dump, const Exec &ex,
+                           const Arg *args, const AttnParams &p, std::string *err);
+
 namespace {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
