@@ -534,7 +534,7 @@ int small_tiles(int d, bool b16, bool causal, bool wave, size_t ws_bytes, const 
     const long R = tiles % cus;
     const size_t fit = R ? ws_bytes / ((size_t)256 * (d + 4) * sizeof(float) * R) : 0;
     const long s = R ? std::min(std::min(cus / R, nb / 2), (long)fit) : 0;
-    const double last = R == 0 ? 0 : s >= 2 ? (double)((nb + s - 1) / s) + (wave ? 7 : 16) / per : (double)nb;
+    const double last = R == 0 ? 0 : s >= 2 ? (double)((nb + s - 1) / s) + (wave ? 13 : 16) / per : (double)nb;
     other = start + per * ((double)(tiles / cus) * nb + last);
   }
   const double one = 5 + (d == 64 ? 0.5e-3 : d == 96 ? 0.7e-3 : 1.0e-3) * steps;
