@@ -40,7 +40,9 @@ class _Arg(ctypes.Structure):  # h3_arg
 
 
 _P, _U64, _U32, _I = ctypes.c_void_p, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_int
-_DISPATCH = (_I, [_P, _P, ctypes.POINTER(_U32), ctypes.POINTER(_U32), ctypes.POINTER(_Arg), _I, _P, _U32, _I, _U32])
+# grid, threads, the h3_arg array and the parameter block travel as plain pointers, so that a launch can pass the bytes
+# of struct.pack as they are
+_DISPATCH = (_I, [_P, _P, _P, _P, _P, _I, _P, _U32, _I, _U32])
 
 # Every exported symbol of include/h3hip.h: (result type, argument types).
 SIGNATURES = {
@@ -186,20 +188,30 @@ class Kernel:
         self.name = f"{file}:{fn}({spec})"
 
 
-def _bind(args) -> tuple:
+# struct format of an array of n h3_arg (buffer handle, byte offset)
+_ARGS = [struct.Struct(f"<{2 * n}Q") for n in range(33)]
+
+
+def _bind(args) -> bytes:
     """The h3_arg array of a launch: a Tensor binds (its buffer, its offset), a (Buffer, offset) pair binds that,
     None binds nothing (a NULL buffer)."""
-    arr = (_Arg * max(1, len(args)))()
-    for slot, a in zip(arr, args):
-        if isinstance(a, Tensor):
-            slot.buf, slot.offset = a.buf.handle, a.offset
-        elif a is not None:
-            slot.buf, slot.offset = a[0].handle, a[1]
-    return arr, len(args)
+    flat = []
+    for a in args:
+        if a is None:
+            flat += (0, 0)
+        elif isinstance(a, Tensor):
+            flat += (a.buf.handle, a.offset)
+        else:
+            flat += (a[0].handle, a[1])
+    try:
+        return _ARGS[len(args)].pack(*flat)
+    except (IndexError, struct.error) as e:
+        raise GpuError(f"cannot bind {len(args)} buffers (at most 32, offsets from 0): {e}") from None
 
 
 def _dims(v):
-    return (_U32 * 3)(*(tuple(v or ()) + (0, 0, 0))[:3])
+    """The three values of a grid or workgroup size, None for NULL (each gfx950 kernel chooses its own)."""
+    return struct.pack("<3I", *(tuple(v) + (0, 0, 0))[:3]) if v else None
 
 
 class Gpu:
@@ -211,14 +223,16 @@ class Gpu:
         self.working_set = lib().h3_recommended_working_set(self.ctx)
         self.max_buffer = lib().h3_max_buffer_length(self.ctx)
         self._kernels = {}
+        self._dispatch, self._static = lib().h3_dispatch, lib().h3_dispatch_static
         self._profile = False
         self.names = []  # in profile mode: the kernel name of each timed launch, in order, until profile_take()
 
     def kernel(self, file: str, fn: str, **macros) -> Kernel:
-        key = (file, fn, tuple(sorted(macros.items())))
-        if key not in self._kernels:
-            self._kernels[key] = Kernel(self, file, fn, macros)
-        return self._kernels[key]
+        key = (file, fn, *macros.items())  # as written: another order of the same macros is another key, the same kernel
+        k = self._kernels.get(key)
+        if k is None:
+            k = self._kernels[key] = Kernel(self, file, fn, macros)
+        return k
 
     def buffer(self, nbytes: int) -> Buffer:
         return Buffer(_call("h3_buffer", self.ctx, max(1, int(nbytes)), fails=_NULL), int(nbytes), self)
@@ -242,11 +256,11 @@ class Gpu:
         `params_index` (default: after the buffers). grid / threads may be None: each gfx950 kernel chooses its own
         geometry from its parameters. no_alloc: the allocation-free entry point (h3_dispatch_static), which uses
         the library's fixed scratch array and is not timed per launch."""
-        arr, n = _bind(args)
-        block = ctypes.create_string_buffer(params, len(params)) if params else None
-        entry = "h3_dispatch_static" if no_alloc else "h3_dispatch"
-        _call(entry, self.ctx, k.handle, _dims(grid), _dims(threads), arr, n, block, len(params),
-              n if params_index is None else params_index, tg_mem)
+        n = len(args)
+        entry = self._static if no_alloc else self._dispatch
+        if entry(self.ctx, k.handle, _dims(grid), _dims(threads), _bind(args), n, params or None, len(params),
+                 n if params_index is None else params_index, tg_mem):
+            raise GpuError(lib().h3_last_error().decode())
         if self._profile and not no_alloc:
             self.names.append(k.name)
 
