@@ -26,12 +26,20 @@
 // consecutive channels per lane: PER = 8 (16-byte loads of 16-bit rows; 16
 // lanes per head at HDIM 128) whenever the rotary pairs (c, c + rot/2) stay
 // lane-aligned (rot/2 a multiple of 8), else the reference's HDIM / 32. Every
-// cross-lane step stays inside the group and runs on DPP lane patterns at 16
-// lanes per slot (ds_swizzle at other shapes; no LDS memory traffic). A workgroup of 256 threads covers 4 waves' groups of slots
-// of 8 consecutive rows; each wave issues all 8 rows' loads before processing
-// them, so enough bytes are in flight to stream HBM, and a slot's 8 scales are
-// stored together. The kernel is HBM-bound: one read of the rows, one write of
-// the codes / values.
+// cross-lane step of the transform and the reductions stays inside the group
+// and runs on DPP lane patterns at 16 lanes per slot (ds_swizzle at other
+// shapes; no LDS memory traffic). A workgroup of 256 threads covers 4 waves'
+// groups of slots of 8 consecutive rows; each wave issues all 8 rows' loads
+// before processing them, and a slot's 8 scales are stored together.
+// With the norm, the rotary embedding, the transform and the int8 rounding the
+// kernel was bound by its vector instructions (about 300 per row and wave,
+// 172-178 us at 16896 rows of 32 + 32 + 32 heads where the bytes take 135), so
+// the work of a row is cut to about 190: what is one value per row (1 / sqrt,
+// the scale and its reciprocal) is computed once for 8 rows, a row per lane;
+// the angle tables of the 8 rows are made once per workgroup in LDS, in
+// channel order, with the rotary signs and the transform's fixed signs folded
+// in; and codes are rounded by one fma each. 150 us (4.7 TB/s) there, 49 -> 44
+// us at 4608 rows; 16-bit outputs 176 -> 152 us.
 #include "h3hip_internal.h"
 
 #include <cmath>
@@ -101,6 +109,31 @@ __device__ __forceinline__ void group_stage(float (&v)[N], float c) {
   }
 }
 
+// the value of lane R of the slot's lane group, on every lane of it
+template <int LPS, int R>
+__device__ __forceinline__ float group_bcast(float v, int gbase) {
+  if constexpr (LPS == 16)  // row_newbcast:R
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + R, 0xF, 0xF, true));
+  else return __shfl(v, gbase + R);
+}
+
+template <int R> using RowConst = std::integral_constant<int, R>;
+// f(RowConst<0>) ... f(RowConst<RPW - 1>): the rows as compile-time constants (a DPP control has to be one)
+template <class F>
+__device__ __forceinline__ void each_row(F &&f) {
+  f(RowConst<0>{}), f(RowConst<1>{}), f(RowConst<2>{}), f(RowConst<3>{});
+  f(RowConst<4>{}), f(RowConst<5>{}), f(RowConst<6>{}), f(RowConst<7>{});
+  static_assert(RPW == 8, "rows");
+}
+
+// QKROT's fixed sign of channel c, as a sign bit
+__device__ __forceinline__ unsigned sign_bit(int c) {
+  return (__builtin_popcount((unsigned)c * 0x2545F491u) & 1u) ? 0x80000000u : 0u;
+}
+__device__ __forceinline__ float flip(float v, unsigned bit) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ bit);
+}
+
 template <int HDIM, int PER, int IN_T, int QK_T, int V_T, bool QKROT>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restrict__ in, const float *__restrict__ wq,
                                                             const float *__restrict__ wk,
@@ -108,29 +141,53 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
                                                             const float *__restrict__ sn, char *__restrict__ Qo,
                                                             char *__restrict__ Ko, char *__restrict__ Vo,
                                                             float *__restrict__ qsc, float *__restrict__ ksc,
-                                                            QkRopeParams p) {
+                                                            QkRopeParams p, int nd) {
   using SH = PrepassShape<HDIM, PER>;
   constexpr int LPS = SH::LPS;
   using IE = typename Elem<IN_T>::type;
   typedef typename VecOf<PER, IE>::type IV;
+  // the rows' angle tables, per channel: cos, and sin with the sign of the channel's half, both times QKROT's sign of
+  // the channel. Channel c at tab_at(c): lanes read 16 consecutive bytes each (PER 8: two runs of 4 channels)
+  __shared__ __attribute__((aligned(16))) float tab[RPW][2][HDIM];
+  auto tab_at = [](int c) { return PER == 8 ? (((c >> 2) & 1) * LPS + (c >> 3)) * 4 + (c & 3) : c; };
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int l32 = lane & (LPS - 1);  // lane within the slot's group
   const int gbase = lane & ~(LPS - 1);  // first lane of the group
   const int g = group_of_lane<LPS>(l32);  // this lane's channel group: channels g * PER .. g * PER + PER - 1
-  const int slot = blockIdx.y * SH::SPG + w * (64 / LPS) + lane / LPS;
-  const int m0 = blockIdx.x * RPW;
+  // Order of the workgroups (nd: slot groups of a row group with int8 outputs, else row groups of a slot group). int8:
+  // a row group's slot groups first, so that the value copies run beside the queries' and keys' arithmetic (16896 rows
+  // of 96 slots: 171 -> 153 us). 16-bit outputs, whose arithmetic is short: the row groups of 4 KB columns first (4608
+  // rows of 72 slots: 31 -> 29 us).
+  constexpr bool ROWS_FIRST = QK_T == T_I8;
+  const int bq = blockIdx.x / nd, br = blockIdx.x - bq * nd;
+  const int bx = ROWS_FIRST ? bq : br, by = ROWS_FIRST ? br : bq;
+  const int slot = by * SH::SPG + w * (64 / LPS) + lane / LPS;
+  const int m0 = bx * RPW;
   const int nslots = p.Hq + p.Hk + p.Hv;
-  if (slot >= nslots) return;  // whole lane groups only; no cross-lane step leaves a group
   const int nr = min(RPW, p.M - m0);
   // outputs are streamed out with nontemporal stores (nothing in this kernel reads them again; measured +6%)
   auto st = [](auto *dst, auto val) { __builtin_nontemporal_store(val, dst); };
 
+  // rows past the last one repeat it and are not stored
   IV xin[RPW];
   {
-    const IE *src = (const IE *)in + (size_t)m0 * p.in_stride + (size_t)slot * HDIM + g * PER;
+    const IE *src = (const IE *)in + (size_t)m0 * p.in_stride + (size_t)min(slot, nslots - 1) * HDIM + g * PER;
 #pragma unroll
     for (int r = 0; r < RPW; r++) xin[r] = *(const IV *)(src + (size_t)min(r, nr - 1) * p.in_stride);
   }
+  const int half_rot = p.rot / 2;
+  if (p.rot && by * SH::SPG < p.Hq + p.Hk) {  // (uniform over the workgroup)
+    for (int i = threadIdx.x; i < nr * p.rot; i += 256) {
+      const int r = i / p.rot, c = i - r * p.rot;
+      const bool first = c < half_rot;
+      const size_t at = (size_t)((m0 + r) % p.seq_len) * half_rot + (first ? c : c - half_rot);
+      const unsigned sb = QKROT ? sign_bit(c) : 0u;
+      tab[r][0][tab_at(c)] = flip(cs[at], sb);
+      tab[r][1][tab_at(c)] = flip(sn[at], sb ^ (first ? 0x80000000u : 0u));
+    }
+    __syncthreads();
+  }
+  if (slot >= nslots) return;  // whole lane groups only; no cross-lane step leaves a group
   const bool isqk = slot < p.Hq + p.Hk, isq = slot < p.Hq;
   const int h = isq ? slot : isqk ? slot - p.Hq : slot - p.Hq - p.Hk;
   const int heads = isq ? p.Hq : isqk ? p.Hk : p.Hv;
@@ -138,66 +195,109 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
     const int sq = m / p.seq_len, r = m - sq * p.seq_len;
     return ((size_t)sq * heads + h) * p.out_rows + r;
   };
-  float keep = 1.0f;  // lane l32 < nr: the scale of row m0 + l32
-  // QKROT's fixed signs: channel c = g * PER + i is negated when popcount(c * 0x2545F491) is odd (its sign
-  // bit, flipped by an xor; computed once per lane)
-  unsigned sbit[PER];
+  if (!isqk) {
+    using OE = typename Elem<V_T>::type;
+    typedef typename VecOf<PER, OE>::type OV;
 #pragma unroll
-  for (int i = 0; i < PER; i++)
-    sbit[i] = (__builtin_popcount((unsigned)(g * PER + i) * 0x2545F491u) & 1u) ? 0x80000000u : 0u;
-
+    for (int rr = 0; rr < RPW; rr++) {
+      if (rr >= nr) break;
+      OE *dst = (OE *)Vo + hrow_of(m0 + rr) * HDIM + g * PER;
+      if constexpr (V_T == IN_T) {
+        st((OV *)dst, xin[rr]);  // same type: a plain copy
+      } else {
+        OV out;
 #pragma unroll
-  for (int rr = 0; rr < RPW; rr++) {
-    if (rr >= nr) break;
-    const int m = m0 + rr;
-    float v[PER];
-#pragma unroll
-    for (int i = 0; i < PER; i++) v[i] = (float)xin[rr][i];
-    const size_t hrow = hrow_of(m);
-    if (isqk) {
-      if (p.norm) {
-        float ss = v[0] * v[0];
-#pragma unroll
-        for (int i = 1; i < PER; i++) ss = ss + v[i] * v[i];
-        // over the groups in halving strides (the partner of group g is g ^ stride)
-        if constexpr (LPS > 16) ss = ss + gshfl<LPS, 16>(ss);
-        if constexpr (LPS > 8) ss = ss + gshfl<LPS, 8>(ss);
-        ss = ss + gshfl<LPS, 4>(ss);
-        ss = ss + gshfl<LPS, 2>(ss);
-        ss = ss + gshfl<LPS, 1>(ss);
-        const float inv = 1.0f / sqrtf(ss / (float)HDIM + p.eps);
-        const float *wv = (isq ? wq : wk) + g * PER;
-#pragma unroll
-        for (int i = 0; i < PER; i++) v[i] = (v[i] * inv) * wv[i];
+        for (int i = 0; i < PER; i++) out[i] = (OE)(float)xin[rr][i];
+        st((OV *)dst, out);
       }
-      if (p.rot) {
-        const int r = m % p.seq_len;
-        const int half_rot = p.rot / 2;
-        const int lanes = half_rot / PER;  // lanes holding the first half of the rotated channels
-        const int src_group = g < lanes ? g + lanes : (g < 2 * lanes ? g - lanes : g);
-        float pv[PER];
+    }
+    return;
+  }
+
+  // What is one value per row (the norm's 1 / sqrt, the int8 scale) is computed once for the 8 rows of a slot: lane r
+  // of the group takes row r's sum (or maximum), and the result is broadcast back row by row.
+  const bool rotated = g * PER < p.rot;  // this lane's channels are in rotary pairs (they then get their signs there)
+  auto sign_of = [&](int i) { return QKROT && !rotated ? sign_bit(g * PER + i) : 0u; };
+  float wv[PER], inv_l = 1.0f;
+  if (p.norm) {
+    const float *ws = (isq ? wq : wk) + g * PER;
 #pragma unroll
-        for (int i = 0; i < PER; i++) pv[i] = __shfl(v[i], gbase + lane_of_group<LPS>(src_group));
-        if (g < 2 * lanes) {
-          const bool first = g < lanes;
-          const int base = (first ? g : g - lanes) * PER;  // pair index of v[0]
-          const float *c = cs + (size_t)r * half_rot + base;
-          const float *s = sn + (size_t)r * half_rot + base;
+    for (int i = 0; i < PER; i++) wv[i] = flip(ws[i], sign_of(i));
+    float mine = 1.0f;
+    each_row([&](auto rc) {
+      constexpr int r = decltype(rc)::value;
+      float ss = (float)xin[r][0] * (float)xin[r][0];
 #pragma unroll
-          for (int i = 0; i < PER; i++) v[i] = first ? v[i] * c[i] - pv[i] * s[i] : v[i] * c[i] + pv[i] * s[i];
+      for (int i = 1; i < PER; i++) ss = ss + (float)xin[r][i] * (float)xin[r][i];
+      // over the groups in halving strides (the partner of group g is g ^ stride)
+      if constexpr (LPS > 16) ss = ss + gshfl<LPS, 16>(ss);
+      if constexpr (LPS > 8) ss = ss + gshfl<LPS, 8>(ss);
+      ss = ss + gshfl<LPS, 4>(ss);
+      ss = ss + gshfl<LPS, 2>(ss);
+      ss = ss + gshfl<LPS, 1>(ss);
+      if (l32 == r) mine = ss;
+    });
+    inv_l = 1.0f / sqrtf(mine / (float)HDIM + p.eps);
+  }
+  const int lanes = half_rot / PER;  // lanes holding the first half of the rotated channels
+  const int src_group = g < lanes ? g + lanes : (g < 2 * lanes ? g - lanes : g);
+  const int from = (gbase + lane_of_group<LPS>(src_group)) * 4;
+  // row r normalised and rotated (and, on QKROT, with its signs)
+  auto row = [&](auto rc, float (&v)[PER]) __attribute__((always_inline)) {
+    constexpr int r = decltype(rc)::value;
+    if (p.norm) {
+      const float inv = group_bcast<LPS, r>(inv_l, gbase);
+#pragma unroll
+      for (int i = 0; i < PER; i++) v[i] = ((float)xin[r][i] * inv) * wv[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < PER; i++) v[i] = flip((float)xin[r][i], sign_of(i));
+    }
+    if (p.rot) {
+      float pv[PER];
+#pragma unroll
+      for (int i = 0; i < PER; i++)
+        pv[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, v[i])));
+      if (rotated) {
+        // v_i c - v_p s on the first half of the channels, v_i c + v_p s on the second (the sign is in the table)
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+          const int at = tab_at(g * PER + i);
+          v[i] = v[i] * tab[r][0][at] + pv[i] * tab[r][1][at];
         }
       }
-      if constexpr (QKROT) {
+    }
+  };
+  if constexpr (QK_T != T_I8) {
+    using OE = typename Elem<QK_T>::type;
+    typedef typename VecOf<PER, OE>::type OV;
+    each_row([&](auto rc) {
+      constexpr int r = decltype(rc)::value;
+      if (r >= nr) return;
+      float v[PER];
+      row(rc, v);
+      OV out;
 #pragma unroll
-        for (int i = 0; i < PER; i++) v[i] = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v[i]) ^ sbit[i]);
+      for (int i = 0; i < PER; i++) out[i] = (OE)v[i];
+      st((OV *)((isq ? Qo : Ko) + (hrow_of(m0 + r) * HDIM + g * PER) * sizeof(OE)), out);
+    });
+  } else {
+    // the transform's final factor 1 / sqrt(HDIM), with the sign that the lane carries (an exact sign change)
+    constexpr float rn = QKROT ? (float)inv_sqrt_hdim<HDIM>() : 1.0f;
+    const float rns = QKROT && (__builtin_popcount(g) & 1) ? -rn : rn;
+    float v[RPW][PER], mine = 0.0f;
+    each_row([&](auto rc) {
+      constexpr int r = decltype(rc)::value;
+      row(rc, v[r]);
+      if constexpr (QKROT) {
 #pragma unroll
         for (int s = 1; s < PER; s <<= 1) {
 #pragma unroll
           for (int i = 0; i < PER; i++) {
             if (!(i & s)) {
-              const float a = v[i], b = v[i + s];
-              v[i] = a + b;
-              v[i + s] = a - b;
+              const float a = v[r][i], b = v[r][i + s];
+              v[r][i] = a + b;
+              v[r][i + s] = a - b;
             }
           }
         }
@@ -206,73 +306,59 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
         // times (-1)^popcount(g) (hadamard_lane_stage)
         auto stage = [&](auto ls_const) {
           constexpr int LS = decltype(ls_const)::value;
-          group_stage<LPS, LS>(v, (g & LS) ? -1.0f : 1.0f);
+          group_stage<LPS, LS>(v[r], (g & LS) ? -1.0f : 1.0f);
         };
         stage(std::integral_constant<int, 1>{});
         stage(std::integral_constant<int, 2>{});
         stage(std::integral_constant<int, 4>{});
         if constexpr (LPS > 8) stage(std::integral_constant<int, 8>{});
         if constexpr (LPS > 16) stage(std::integral_constant<int, 16>{});
-        // the sign carried by the lane goes into the final scale (an exact sign change of the same product)
-        constexpr float rn = (float)inv_sqrt_hdim<HDIM>();
-        const float rns = (__builtin_popcount(g) & 1) ? -rn : rn;
-#pragma unroll
-        for (int i = 0; i < PER; i++) v[i] *= rns;
       }
-      if constexpr (QK_T == T_I8) {
-        float amax = 0.0f;
+      float amax = 0.0f;
 #pragma unroll
-        for (int i = 0; i < PER; i++) amax = fmaxf(amax, fabsf(v[i]));
-        if constexpr (LPS > 16) amax = fmaxf(amax, gshfl<LPS, 16>(amax));
-        if constexpr (LPS > 8) amax = fmaxf(amax, gshfl<LPS, 8>(amax));
-        amax = fmaxf(amax, gshfl<LPS, 4>(amax));
-        amax = fmaxf(amax, gshfl<LPS, 2>(amax));
-        amax = fmaxf(amax, gshfl<LPS, 1>(amax));
-        const float scale = amax > 0.0f ? amax / 127.0f : 1.0f;
-        const float rs = __builtin_amdgcn_rcpf(scale);  // 1 ulp
-        typedef typename VecOf<PER, signed char>::type CV;
-        CV codes;
+      for (int i = 0; i < PER; i++) amax = fmaxf(amax, fabsf(v[r][i]));
+      if constexpr (LPS > 16) amax = fmaxf(amax, gshfl<LPS, 16>(amax));
+      if constexpr (LPS > 8) amax = fmaxf(amax, gshfl<LPS, 8>(amax));
+      amax = fmaxf(amax, gshfl<LPS, 4>(amax));
+      amax = fmaxf(amax, gshfl<LPS, 2>(amax));
+      amax = fmaxf(amax, gshfl<LPS, 1>(amax));
+      if (l32 == r) mine = amax;
+    });
+    // rounding is monotonic, so the largest |v * rn| is the rounded product of the largest |v|
+    const float am = QKROT ? mine * rn : mine;
+    const float scale_l = am > 0.0f ? am / 127.0f : 1.0f;
+    const float rs_l = __builtin_amdgcn_rcpf(scale_l);  // 1 ulp
+    each_row([&](auto rc) {
+      constexpr int r = decltype(rc)::value;
+      if (r >= nr) return;
+      // Codes are the nearest integers of fl(v * rns) / scale. y = v * (rns * rs) is within 2^-14 of that quotient
+      // (|y| <= 128; four roundings of at most 1 ulp), so their nearest integers agree unless y lies within 2^-14 of
+      // a half-integer, and then the wave divides (one row of four slots in sixteen, and exact). t = fma(v, f, 1.5 * 2^23) rounds y to
+      // the nearest integer (half to even), whose two's complement is in t's low bits. A scale whose reciprocal is not
+      // a normal float (amax below ~2^-119) divides too, and so does a NaN (`far` keeps it).
+      const float rs = group_bcast<LPS, r>(rs_l, gbase), f = rs * rns;
+      constexpr float MG = 12582912.0f;
+      unsigned t[PER];
+      float far = 0.0f;
 #pragma unroll
-        for (int i = 0; i < PER; i++) codes[i] = (signed char)(int)rintf(v[i] * rs);
-        // |v / scale| <= 127.5 and rs is within 1 ulp of 1/scale, so v * rs is within 2^-16 + 2^-18 < 2^-15 of
-        // the exact quotient: its nearest integer is the quotient's unless it lies within 2^-15 of a
-        // half-integer, and then the lanes concerned divide (rare, and exact). A scale whose reciprocal is not
-        // a normal float (amax below ~2^-119) divides on every lane.
-        bool near_half = !(rs < 0x1p126f);
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-          const float y = v[i] * rs;
-          near_half |= fabsf(y - rintf(y)) > 0.5f - 0x1p-15f;
-        }
-        if (near_half) {
-#pragma unroll
-          for (int i = 0; i < PER; i++) codes[i] = (signed char)(int)rintf(v[i] / scale);
-        }
-        st((CV *)((isq ? Qo : Ko) + hrow * HDIM + g * PER), codes);
-        if (l32 == rr) keep = scale;
-      } else {
-        using OE = typename Elem<QK_T>::type;
-        typedef typename VecOf<PER, OE>::type OV;
-        OV out;
-#pragma unroll
-        for (int i = 0; i < PER; i++) out[i] = (OE)v[i];
-        st((OV *)((isq ? Qo : Ko) + (hrow * HDIM + g * PER) * sizeof(OE)), out);
+      for (int i = 0; i < PER; i++) {
+        const float ti = __builtin_fmaf(v[r][i], f, MG);
+        far = __builtin_elementwise_maximum(far, fabsf(__builtin_fmaf(v[r][i], f, -(ti - MG))));
+        t[i] = __builtin_bit_cast(unsigned, ti);
       }
-    } else {
-      using OE = typename Elem<V_T>::type;
-      typedef typename VecOf<PER, OE>::type OV;
-      if constexpr (V_T == IN_T) {
-        st((OV *)(Vo + (hrow * HDIM + g * PER) * sizeof(OE)), xin[rr]);  // same type: a plain copy
-      } else {
-        OV out;
+      // wave-uniform, so that the broadcast's source lanes are active
+      if (__builtin_amdgcn_ballot_w64(!(far <= 0.5f - 0x1p-14f) || !(rs < 0x1p126f))) {
+        const float scale = group_bcast<LPS, r>(scale_l, gbase);
 #pragma unroll
-        for (int i = 0; i < PER; i++) out[i] = (OE)v[i];
-        st((OV *)(Vo + (hrow * HDIM + g * PER) * sizeof(OE)), out);
+        for (int i = 0; i < PER; i++) t[i] = (unsigned)(int)rintf((QKROT ? v[r][i] * rns : v[r][i]) / scale);
       }
-    }
-  }
-  if constexpr (QK_T == T_I8) {
-    if (isqk && l32 < nr) (isq ? qsc : ksc)[hrow_of(m0 + l32)] = keep;
+      typedef typename VecOf<PER, signed char>::type CV;
+      CV codes;
+#pragma unroll
+      for (int i = 0; i < PER; i++) codes[i] = (signed char)t[i];
+      st((CV *)((isq ? Qo : Ko) + hrow_of(m0 + r) * HDIM + g * PER), codes);
+    });
+    if (l32 < nr) (isq ? qsc : ksc)[hrow_of(m0 + l32)] = scale_l;
   }
 }
 
@@ -355,11 +441,12 @@ int launch_qk(const Pipeline &pl, const Exec &ex, const Arg *a, int nargs, const
   auto go = [&](auto per_const) {
     constexpr int P = decltype(per_const)::value;
     constexpr int SPG = PrepassShape<HDIM, P>::SPG;
-    dim3 grid((unsigned)((p.M + RPW - 1) / RPW), (unsigned)((nslots + SPG - 1) / SPG));
+    const int nx = (p.M + RPW - 1) / RPW, ny = (nslots + SPG - 1) / SPG;
+    const dim3 grid((unsigned)nx * ny);
     hipLaunchKernelGGL((qk_norm_rope_kernel<HDIM, P, IN_T, QK_T, V_T, QKROT>), grid, dim3(256), 0, ex.stream, a[0].ptr,
                        (const float *)a[1].ptr, (const float *)a[2].ptr, (const float *)a[3].ptr,
                        (const float *)a[4].ptr, a[5].ptr, a[6].ptr, a[7].ptr,
-                       nargs > 9 ? (float *)a[9].ptr : nullptr, nargs > 10 ? (float *)a[10].ptr : nullptr, p);
+                       nargs > 9 ? (float *)a[9].ptr : nullptr, nargs > 10 ? (float *)a[10].ptr : nullptr, p, QK_T == T_I8 ? ny : nx);
   };
   if ((p.rot / 2) % 8 == 0) go(std::integral_constant<int, 8>{});
   else go(std::integral_constant<int, HDIM / 32>{});

@@ -320,3 +320,20 @@ def test_per_stream_row_offset_views(gpu):
     assert np.array_equal(qs.numpy().view(np.uint32), want["qs"].view(np.uint32))
     assert np.array_equal(ks.numpy().view(np.uint32), want["ks"].view(np.uint32))
     assert np.array_equal(V.numpy(), to_bf16(want["V"]))
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_codes_at_half_integers(gpu, hd):
+    """Quotients exactly at and one ulp either side of half-integers (scale 1 and a power of two), where the fast
+    rounding has to hand over to the division: codes bit for bit (half to even)."""
+    M, H = 21, 3
+    n = np.arange(M * 3 * H * hd) % 251 - 125 + 0.5
+    x = n.astype(np.float32).reshape(M, 3, H, hd)
+    x[1::3], x[2::3] = np.nextafter(x[1::3], np.float32(np.inf)), np.nextafter(x[2::3], np.float32(-np.inf))
+    x[..., 5] = 127  # the largest magnitude of every row
+    x[M // 2:] *= 2.0 ** -9
+    x = x.reshape(M, 3 * H * hd)
+    got = run_prepass(gpu, x, "f32", M=M, Hq=H, Hk=H, Hv=H, hd=hd, out_rows=64, qk_rot=False)
+    want = op.qk_norm_rope(x, Hq=H, Hk=H, Hv=H, hd=hd, out_rows=64, rot=0, eps=1e-6, norm=False, q8=True, qk_rot=False)
+    for n in ("Q", "K", "qs", "ks"):
+        assert np.array_equal(got[n][:, :M], want[n][:, :M]), n
