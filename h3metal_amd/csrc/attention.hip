@@ -530,7 +530,8 @@ int small_tiles(int d, bool b16, bool causal, bool wave, size_t ws_bytes, const 
     for (long t = 0; t < nqb; t++) total += (double)((keys(256 * t + 256) + BK - 1) / BK) * p.H;
     other = 5 + 2.2 * std::max((double)((keys(256 * nqb) + BK - 1) / BK), total / cus);
   } else {
-    const double start = wave ? (b16 ? 12 : 15) : 5, per = wave ? (b16 ? 1.55 : 1.8) : d == 128 ? 2.2 : 1.65;
+    const double start = wave ? (b16 ? 12 : 15) : d == 64 ? 3 : 5;
+    const double per = wave ? (b16 ? 1.55 : 1.8) : d == 128 ? 2.2 : d == 96 ? 1.65 : 1.5;
     const long R = tiles % cus;
     const size_t fit = R ? ws_bytes / ((size_t)256 * (d + 4) * sizeof(float) * R) : 0;
     const long s = R ? std::min(std::min(cus / R, nb / 2), (long)fit) : 0;
