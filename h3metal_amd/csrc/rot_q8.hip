@@ -44,6 +44,26 @@ template <int N, typename E> struct VecOf { typedef E type __attribute__((ext_ve
 
 constexpr int RB = 256;  // rotation block
 
+// g / (1 + exp(-g)) in float, from e = exp(-|g|) <= 1 (no overflow): g / (1 + e), or g e / (1 + e) for negative g. The
+// exponent |g| log2(e) is taken with its rounding error and the constant's second part, put back to first order (they
+// are below 2^-15); the quotient by 1 + e, in [1, 2], from the hardware reciprocal and one step on its
+// remainder. div_fixup gives infinities and NaN what the division gives them. The gated kernel is bound by its vector
+// instructions; expf and the compiler's division took 40 of its issue slots a value, this takes 25: 16896 rows of 4096
+// columns 92 -> 80 us. The scales' error against 64 bits is 1% smaller (5.34e-8 against 5.42e-8 over six inputs).
+__device__ __forceinline__ float silu(float g) {
+  constexpr float L = 1.44269504088896340736f, L2 = 1.92596303e-8f, LN2 = 0.693147180559945309417f;
+  const float a = fminf(fabsf(g), 200.0f);  // exp(-200) is zero
+  const float t = a * -L;
+  const float lo = __builtin_fmaf(a, -L2, __builtin_fmaf(a, -L, -t));
+  const float e0 = __builtin_amdgcn_exp2f(t);
+  const float e = __builtin_fmaf(e0, lo * LN2, e0);
+  const float d = 1.0f + e, num = g < 0.0f ? g * e : g;
+  const float r = __builtin_amdgcn_rcpf(d), q = num * r;
+  // the remainder num - (1 + e) q, with what the sum lost (d - 1 is exact, and so is the difference)
+  const float rem = __builtin_fmaf(-(e - (d - 1.0f)), q, __builtin_fmaf(-d, q, num));
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(rem, r, q), d, num);
+}
+
 template <int IN_T, bool SWIGLU, bool OUT_HR, int MAXB>
 __global__ __launch_bounds__(256) void rot_q8_kernel(const char *__restrict__ in, char *__restrict__ out,
                                                       float *__restrict__ sa, RotQParams p) {
@@ -76,7 +96,7 @@ __global__ __launch_bounds__(256) void rot_q8_kernel(const char *__restrict__ in
       float val = (float)xv[b][i];
       if constexpr (SWIGLU) {
         const float g = (float)xg[b][i];
-        val = val * (g / (1.0f + expf(-g)));
+        val = val * silu(g);
       }
       v[b][i] = val;
     }
@@ -141,9 +161,11 @@ __global__ __launch_bounds__(256) void rot_q8_kernel(const char *__restrict__ in
     for (int b = 0; b < MAXB; b++) {
       const int blk = hw + 8 * b;
       if (blk < nb) {
+        // |v rs| <= 127.5: adding 1.5 * 2^23 rounds to the nearest integer (half to even), whose two's complement is
+        // then in the low bits
         c8 cv;
 #pragma unroll
-        for (int i = 0; i < 8; i++) cv[i] = (signed char)(int)rintf(v[b][i] * rs);
+        for (int i = 0; i < 8; i++) cv[i] = (signed char)__builtin_bit_cast(unsigned, v[b][i] * rs + 12582912.0f);
         *(c8 *)(o + blk * RB + l32 * 8) = cv;
       }
     }
