@@ -154,13 +154,9 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
   const int l32 = lane & (LPS - 1);  // lane within the slot's group
   const int gbase = lane & ~(LPS - 1);  // first lane of the group
   const int g = group_of_lane<LPS>(l32);  // this lane's channel group: channels g * PER .. g * PER + PER - 1
-  // Order of the workgroups (nd: slot groups of a row group with int8 outputs, else row groups of a slot group). int8:
-  // a row group's slot groups first, so that the value copies run beside the queries' and keys' arithmetic (16896 rows
-  // of 96 slots: 171 -> 153 us). 16-bit outputs, whose arithmetic is short: the row groups of 4 KB columns first (4608
-  // rows of 72 slots: 31 -> 29 us).
-  constexpr bool ROWS_FIRST = QK_T == T_I8;
-  const int bq = blockIdx.x / nd, br = blockIdx.x - bq * nd;
-  const int bx = ROWS_FIRST ? bq : br, by = ROWS_FIRST ? br : bq;
+  // order of the workgroups: nd > 0 row groups of a slot group first, or -nd slot groups of a row group first (launch_qk)
+  const int nn = nd > 0 ? nd : -nd, bq = blockIdx.x / nn, br = blockIdx.x - bq * nn;
+  const int bx = nd > 0 ? br : bq, by = nd > 0 ? bq : br;
   const int slot = by * SH::SPG + w * (64 / LPS) + lane / LPS;
   const int m0 = bx * RPW;
   const int nslots = p.Hq + p.Hk + p.Hv;
@@ -443,10 +439,16 @@ int launch_qk(const Pipeline &pl, const Exec &ex, const Arg *a, int nargs, const
     constexpr int SPG = PrepassShape<HDIM, P>::SPG;
     const int nx = (p.M + RPW - 1) / RPW, ny = (nslots + SPG - 1) / SPG;
     const dim3 grid((unsigned)nx * ny);
+    // The order of the workgroups. int8 calls whose rows outgrow the 256 MB last-level cache together with the outputs
+    // run a row group's slot groups first, so that the value copies overlap the queries' and keys' arithmetic (415 MB
+    // of rows: 171 -> 153 us, 201 MB: 82 -> 76). Otherwise the row groups of a slot group's 4 KB columns go first
+    // (113 MB of rows just written by a projection: 50 -> 45 us, 37 MB: 23 -> 20; 16-bit outputs 31 -> 29 at 85 MB).
+    const bool rows_first = QK_T == T_I8 && (uint64_t)p.M * nslots * HDIM * esize(IN_T) > 160000000ull;
     hipLaunchKernelGGL((qk_norm_rope_kernel<HDIM, P, IN_T, QK_T, V_T, QKROT>), grid, dim3(256), 0, ex.stream, a[0].ptr,
                        (const float *)a[1].ptr, (const float *)a[2].ptr, (const float *)a[3].ptr,
                        (const float *)a[4].ptr, a[5].ptr, a[6].ptr, a[7].ptr,
-                       nargs > 9 ? (float *)a[9].ptr : nullptr, nargs > 10 ? (float *)a[10].ptr : nullptr, p, QK_T == T_I8 ? ny : nx);
+                       nargs > 9 ? (float *)a[9].ptr : nullptr, nargs > 10 ? (float *)a[10].ptr : nullptr, p,
+                       rows_first ? -ny : nx);
   };
   if ((p.rot / 2) % 8 == 0) go(std::integral_constant<int, 8>{});
   else go(std::integral_constant<int, HDIM / 32>{});
