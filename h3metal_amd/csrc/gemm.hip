@@ -55,13 +55,6 @@ using TileSmall = GTile<128, 128>;
 // 16-byte piece p of LDS row r (64 bytes) sits at slot p ^ ((r / 4) % 4)
 __device__ __forceinline__ int swz(int row, int piece) { return row * KS + ((piece ^ ((row >> 2) & 3)) << 4); }
 
-template <int OT>
-__device__ __forceinline__ void store_out(char *p, float v) {
-  if constexpr (OT == T_F32) *(float *)p = v;
-  else if constexpr (OT == T_BF16) *(__bf16 *)p = (__bf16)v;
-  else *(_Float16 *)p = (_Float16)v;
-}
-
 template <int OT, int EPI, bool HAS_BIAS, int AT, int SM, class TL>
 __global__ __launch_bounds__(NWG * 64) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(const char *__restrict__ A,
                                                            const char *__restrict__ W,

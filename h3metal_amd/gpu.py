@@ -35,10 +35,6 @@ def _find_library() -> str:
     raise FileNotFoundError(f"{LIB_NAME} not found next to {__file__}; build it with `python -m h3metal_amd.build`")
 
 
-class _Arg(ctypes.Structure):  # h3_arg
-    _fields_ = [("buf", ctypes.c_void_p), ("offset", ctypes.c_uint64)]
-
-
 _P, _U64, _U32, _I = ctypes.c_void_p, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_int
 # grid, threads, the h3_arg array and the parameter block travel as plain pointers, so that a launch can pass the bytes
 # of struct.pack as they are
