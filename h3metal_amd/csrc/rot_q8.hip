@@ -159,18 +159,24 @@ __global__ __launch_bounds__(256) void rot_q8_kernel(const char *__restrict__ in
     const float rs = 1.0f / scale;
     typedef signed char c8 __attribute__((ext_vector_type(8)));
     char *o = out + (size_t)m * p.D;
+    auto store = [&](auto code) __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < MAXB; b++) {
-      const int blk = hw + 8 * b;
-      if (blk < nb) {
-        // |v rs| <= 127.5: adding 1.5 * 2^23 rounds to the nearest integer (half to even), whose two's complement is
-        // then in the low bits
-        c8 cv;
+      for (int b = 0; b < MAXB; b++) {
+        const int blk = hw + 8 * b;
+        if (blk < nb) {
+          c8 cv;
 #pragma unroll
-        for (int i = 0; i < 8; i++) cv[i] = (signed char)__builtin_bit_cast(unsigned, v[b][i] * rs + 12582912.0f);
-        *(c8 *)(o + blk * RB + l32 * 8) = cv;
+          for (int i = 0; i < 8; i++) cv[i] = code(v[b][i] * rs);
+          *(c8 *)(o + blk * RB + l32 * 8) = cv;
+        }
       }
-    }
+    };
+    // |v rs| <= 127.5: adding 1.5 * 2^23 rounds to the nearest integer (half to even), whose two's complement is then
+    // in the low bits. Not so where 1 / scale overflows (amax below 127 * 2^-128; the same for the whole row), and a NaN
+    // of 32-bit rows may carry payload bits there (one of 16-bit rows has none so low): those are converted, so that a
+    // NaN has code 0.
+    if (IN_T == T_F32 || rs == INFINITY) store([](float y) { return (signed char)(int)rintf(y); });
+    else store([](float y) { return (signed char)__builtin_bit_cast(unsigned, y + 12582912.0f); });
     if (threadIdx.x == 0) sa[m] = scale;
   }
 }

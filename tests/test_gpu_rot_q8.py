@@ -64,6 +64,31 @@ def test_tiny_and_large_rows_bit_exact(gpu, mag, dt):
     assert np.array_equal(codes, wc)
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+def test_codes_of_nan_and_of_rows_whose_reciprocal_overflows(gpu, dt):
+    """A block with a NaN (with payload bits as low as the type holds) has code 0 throughout, and the other blocks of
+    the row are coded as without it. A row with amax below 127 * 2^-128, whose 1 / scale is infinite, has quotients of
+    +-infinity and, at zeros, NaN: their codes are the low bytes of the saturated conversion, -1, 0 and 0."""
+    rng = np.random.default_rng(15)
+    M, D = 3, 768
+    xh, xf = host_rows(rng, M, D, dt)
+    nan = {"f32": np.uint32(0x7FC00055), "bf16": np.uint16(0x7FD5), "f16": np.uint16(0x7E55)}[dt]
+    xh[1, 300:302].view(nan.dtype)[:] = nan
+    codes, sa = run_rot(gpu, xh, dt, M, D)
+    xf[1, 256:512] = 0
+    wc, ws, _ = orq.rot_q8(xf, D)
+    assert np.array_equal(sa.view(np.uint32), ws.view(np.uint32))
+    assert np.array_equal(codes, wc)
+    if dt == "f16":
+        return  # no such small values
+    x = np.zeros((1, D), np.float32)
+    x[0, 3] = 2.0 ** -125  # one-hot: the rotated block is +-2^-129
+    codes, sa = run_rot(gpu, to_bf16(x) if dt == "bf16" else x, dt, 1, D)
+    r = orq.rotate_rows_f32(x)
+    assert sa[0] == np.abs(r).max() / np.float32(127) and 1 / float(sa[0]) > 2.0 ** 128
+    assert np.array_equal(codes, np.where(r > 0, -1, 0).astype(np.int8))
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_random_shape_sweep_bit_exact(gpu, seed):
     """A seeded sweep: widths of 1 to 56 Hadamard blocks of 256, up to 3000 rows, three input types, some rows
