@@ -45,8 +45,10 @@ template <> struct Elem<T_F32> { using type = float; };
 template <int N, typename E> struct VecOf { typedef E type __attribute__((ext_vector_type(N))); };
 
 constexpr int RB = 256;  // rotation block
+constexpr float SILU_MIN = -87.0f;  // the lowest gate of silu()
 
-// g / (1 + exp(-g)) in float, from e = exp(-|g|) <= 1 (no overflow): g / (1 + e), or g e / (1 + e) for negative g. The
+// g / (1 + exp(-g)) in float, from e = exp(-|g|) <= 1 (no overflow): g / (1 + e), or g e / (1 + e) for negative g (from
+// SILU_MIN; lower gates are computed by the caller). The
 // exponent |g| log2(e) is taken with its rounding error and the constant's second part, put back to first order (they
 // are below 2^-15); the quotient by 1 + e, in [1, 2], from the hardware reciprocal and one step on its
 // remainder. div_fixup gives infinities and NaN what the division gives them. The gated kernel is bound by its vector
@@ -96,11 +98,25 @@ __global__ __launch_bounds__(256) void rot_q8_kernel(const char *__restrict__ in
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       float val = (float)xv[b][i];
-      if constexpr (SWIGLU) {
-        const float g = (float)xg[b][i];
-        val = val * silu(g);
-      }
+      if constexpr (SWIGLU) val = val * silu((float)xg[b][i]);
       v[b][i] = val;
+    }
+    if constexpr (SWIGLU) {
+      // silu's exp(-|g|) is subnormal below -87.33, and the hardware exponential flushes it: gates below SILU_MIN, told
+      // by their sign and magnitude bits, take the library's exp and division (a normal float down to -88.7)
+      unsigned far = 0;
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const unsigned bits = __builtin_bit_cast(unsigned, (float)xg[b][i]);
+        far = far > bits ? far : bits;
+      }
+      if (far > __builtin_bit_cast(unsigned, SILU_MIN)) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const float g = (float)xg[b][i];
+          if (g < SILU_MIN) v[b][i] = (float)xv[b][i] * (g / (1.0f + expf(-g)));
+        }
+      }
     }
     // columns 8 l32 + i: bits 0-2 in the lane, bits 3-7 across lanes
 #pragma unroll

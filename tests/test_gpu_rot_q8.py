@@ -129,6 +129,41 @@ def test_swiglu_within_one_code(gpu):
     assert (codes != wc).mean() < 1e-3
 
 
+GATES = [0.0, -0.0, 1e-30, -1e-30, 0.5, -0.5, 20.0, -20.0, -86.5, 87.0, -87.0, -87.25, -87.5, 88.0, -88.0, -88.5, 89.0,
+         -89.0, 200.0, -200.0, 1e4, -1e4, np.inf, -np.inf, np.nan]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_swiglu_gates_over_the_float_range(gpu, dt):
+    """One gate per 256-column block (every other column of it zero), its value scaled so that the product is near
+    16 where that is possible: the rotated block is a 16th of it. Gates to -88.5 (exp(-g) is finite to -88.7) are held to
+    2^-10, twice the rounding of the half output; below, g / (1 + exp(-g)) is zero in float. Infinities and NaN
+    give what the formula gives (-inf / inf is NaN)."""
+    D = 256 * len(GATES)
+    x = np.zeros((1, 2 * D), np.float32)
+    g = np.array(GATES, np.float32)
+    g = from_bf16(to_bf16(g)) if dt == "bf16" else g
+    with np.errstate(all="ignore"):
+        f = g.astype(np.float64) / (1 + np.exp(-g.astype(np.float64)))
+        small = np.isfinite(f) & (np.abs(f) > 1e-37)
+        val = np.where(small, 16 / np.where(small, f, 1), 1.0).clip(-3e38, 3e38).astype(np.float32)
+    val = from_bf16(to_bf16(val))
+    x[0, 0:D:256], x[0, D::256] = val, g
+    xh = to_bf16(x) if dt == "bf16" else x
+    out, _ = run_rot(gpu, xh, dt, 1, D, swiglu=True, out_hr=True)
+    out = out.reshape(len(GATES), 256).astype(np.float64)
+    with np.errstate(all="ignore"):
+        want = orq.silu_gated_f32(np.concatenate([val, g])[None], len(GATES))[0].astype(np.float64) / 16
+    for i, gate in enumerate(GATES):
+        w = np.full(256, want[i])  # column 0 is the Hadamard matrix's row of ones
+        if np.isnan(want[i]):
+            assert np.isnan(out[i]).all(), gate
+        elif np.isinf(want[i]) or want[i] == 0:
+            assert np.array_equal(out[i], w), gate
+        else:
+            assert np.abs(out[i] / w - 1).max() < 2 ** -10, (gate, out[i][0], want[i])
+
+
 def test_reference_tolerance_case(gpu):
     """tests/test_ops.py::test_rot at its own shape (M=19, D=14336, swiglu, bf16 input): dequantised rows within
     0.6/127 of the float64 rotation (relative to the row maximum), the rotated half output within 2e-3."""
