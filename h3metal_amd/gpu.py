@@ -207,7 +207,7 @@ def _bind(args) -> bytes:
 
 def _dims(v):
     """The three values of a grid or workgroup size, None for NULL (each gfx950 kernel chooses its own)."""
-    return struct.pack("<3I", *(tuple(v) + (0, 0, 0))[:3]) if v else None
+    return (_U32 * 3)(*(tuple(v) + (0, 0, 0))[:3]) if v else None
 
 
 class Gpu:

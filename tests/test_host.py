@@ -39,6 +39,14 @@ def test_open_without_gpu_fails_cleanly():
         G.Gpu()
 
 
+def test_launch_geometry_is_taken_as_32_bit_words():
+    """A grid or workgroup size of up to three values, None or empty for NULL; the kernels choose their own geometry, so
+    values past 32 bits are cut to them and not refused."""
+    assert G._dims(None) is None and G._dims(()) is None
+    assert list(G._dims((7,))) == [7, 0, 0] and list(G._dims([1, 2, 3, 4])) == [1, 2, 3]
+    assert list(G._dims((1 << 32, -1, (1 << 33) + 5))) == [0, 0xFFFFFFFF, 5]
+
+
 class FakeGpu:
     """Records what a launcher asks the runtime for."""
 
