@@ -505,42 +505,101 @@ size_t attention_workspace_max(int cus) { return (size_t)std::max(cus, 1) * 384 
 
 namespace {
 
-// Whether a call runs on the small tiles of attention_small.hip: 0 no, else the 32-row query tiles per workgroup (1 or
-// 2). Decided by the estimated time (us) of both, from a sweep on an MI355X (head counts 4 to 512, 64 to 5000 rows,
-// head dims 64, 96, 128, int8 and 16-bit scores, causal and not):
-//  small tiles: 5 + c us per 1000 (32-query, 32-key) blocks, c = 0.5, 0.7, 1.0 for head dim 64, 96, 128 (two query tiles
-//  per workgroup at head dim 96: 12 + 0.95 per 1000 (64, 32) blocks, less from about 50 000 blocks on);
-//  256-row tiles: a start plus a time per 64-key block of each round of workgroups, plus the merge of a split last
-//  round. With a causal mask the longest tile or the mean load of a CU.
-// Measured, 256-row -> small tiles: bf16 H 4 256 rows 15.7 -> 9.0, int8 H 32 600 rows 33.8 -> 19.5 (1300: 58.9 -> 53.1,
-// 1800: 70 against 90, not taken), causal H 32 512 rows 24.7 -> 11.2, head dim 96 H 16 1037 rows 33.3 -> 22.8 (3000: 78
-// against 82, not taken), head dim 64 H 128 256 rows 26.8 -> 9.8. The small tiles have to be estimated 7% faster.
-int small_tiles(int d, bool b16, bool causal, bool wave, const AttnParams &p) {
+// Estimated times (us) that choose between 256-row tiles (this file's kernel, the wave-pipelined one at head dim 128
+// without a causal mask) and the small tiles of attention_small.hip. Fitted to 3200 calls on an MI355X, timed on every kernel that
+// can run them: head dims 64, 96, 128, 8-bit and 16-bit scores, 1 to 512 heads, 1 to 5000 queries, 1 to 60 000 keys,
+// causal with offsets up to 30 000 and not. Error of the fits: 256-row tiles 5% on average and 1.6x at worst, small tiles
+// 6% and 2.3x (hundreds of heads whose K and V come from memory once).
+struct WholeTimes {
+  // without a causal mask: a start, a 64-key block, a full round of workgroups, their rows (256 of a tile), and what a
+  // split last round adds: fixed, per unit (a chunk of a tile) with 256 rows, per chunk of a tile (the merge reads them
+  // one after another), per unit
+  double start, block, round, rows, split, unit_rows, chunk, unit;
+  // with one: a start, a block of the longest tile, or a block and a tile of a CU's mean load
+  double c_start, c_longest, c_block, c_tile;
+};
+struct SmallTimes {
+  // a start, a round of workgroups, and a wave's block (a quarter of the keys, 32 at a time) where 1 .. `slots` (what LDS
+  // and registers hold) workgroups share a CU
+  int slots;
+  double start, round, block[4];
+  double c_start, c_longest, c_block, c_tile;  // as above, a block of a wave
+};
+constexpr WholeTimes WHOLE[3][2] = {  // head dim 64, 96, 128; 16-bit, 8-bit scores
+    {{4.1, 1.1, 0.93, 2.8, 2.6, 0.03, 0.19, 0.018, 4.4, 1.8, 2.8, -0.9},
+     {4.2, 1.3, 1.0, 2.5, 2.6, 0.027, 0.19, 0.021, 4.2, 2.2, 3.3, -1.3}},
+    {{3.5, 1.6, 1.5, 4.5, 3.6, 0.038, 0.42, 0.026, 4.7, 1.9, 2.9, -0.93},
+     {3.9, 1.4, 1.8, 4.2, 3.8, 0.035, 0.42, 0.029, 4.4, 2.3, 3.5, -1.0}},
+    {{5.0, 1.5, 3.9, 7.7, 5.8, 0.028, 0.22, 0.032, 5.0, 1.9, 3.1, -1.1},
+     {4.1, 1.3, 2.2, 8.0, 5.8, 0.027, 0.22, 0.033, 4.4, 2.3, 3.6, -0.93}}};
+constexpr SmallTimes SMALL[4][2] = {  // head dim 64, 96, 128; 96 with two query tiles per workgroup
+    {{4, 3.5, 1.6, {0.41, 0.71, 0.94, 1.5}, 4.9, 0.44, 0.4, 0.55},
+     {4, 3.4, 1.8, {0.43, 0.63, 0.82, 1.1}, 5.9, 0.34, 0.34, 0.41}},
+    {{2, 2.7, 2.3, {0.56, 1.1}, 5.1, 0.58, 0.63, 1.2}, {3, 2.5, 2.6, {0.54, 0.98, 1.2}, 5.7, 0.51, 0.49, 0.91}},
+    {{2, 1.5, 3.4, {0.6, 1.2}, 5.1, 0.61, 0.73, 1.6}, {2, 1.6, 3.4, {0.61, 0.95}, 5.6, 0.59, 0.55, 1.6}},
+    {{2, 1.2, 4.4, {0.88, 1.8}, 5.7, 0.89, 1.0, 2.1}, {2, 0.88, 4.8, {0.9, 1.5}, 5.7, 0.94, 0.85, 2.3}}};
+
+// Key blocks of the n tiles of a causal call, tile t (from 1) with the keys before `rows` t + off, at most L, in blocks of
+// `blk` (a divisor of `rows`): their sum, and the longest tile's
+struct CausalBlocks {
+  double sum, longest;
+};
+CausalBlocks causal_blocks(long n, long rows, long blk, long off, long L) {
+  const long k = rows / blk, c = off >= 0 ? (off + blk - 1) / blk : -(-off / blk), top = (L + blk - 1) / blk;
+  // tiles first .. past - 1 have k t + c blocks, earlier ones none and later ones `top`
+  const long first = std::min(c < 0 ? -c / k + 1 : 1L, n + 1);
+  const long past = std::max(first, std::min(top > c ? (top - c + k - 1) / k : 1L, n + 1)), m = past - first;
+  const double sum = 0.5 * k * (first + past - 1) * m + (double)c * m + (double)top * (n + 1 - past);
+  return {sum, (double)std::max(0L, std::min(top, k * n + c))};
+}
+
+// Whether a call runs on the small tiles: 0 no, else the 32-row query tiles per workgroup (1, or 2 at head dim 96). They
+// have to be estimated 5% faster than the 256-row tiles, and two query tiles 5% faster than one. Over the calls above the
+// choice costs 0.4% on average against the best kernel of each (1.39x at worst), and 7 of them are over 5% slower than on
+// 256-row tiles (1.19x at worst). An estimate without the chain of a workgroup's key blocks took 313 such calls, short
+// queries against long keys (int8, 4 heads, 32 queries, 32 768 keys: 43 us on 256-row tiles, 163 on small ones).
+// Measured, 256-row -> small tiles: bf16 H 4 256 rows 15.2 -> 6.1, int8 H 24 600 rows 27.0 -> 10.8, causal H 32 512 rows
+// 24.0 -> 11.4, head dim 96 H 16 1037 rows 31.9 -> 20.5, head dim 64 H 128 200 rows 24.4 -> 8.5.
+int small_tiles(int d, bool q8, bool causal, const AttnParams &p) {
   const long cus = cu_count();
-  if (cus <= 0 || (uint64_t)(p.L + 256) * d * 2 > 0x7fffffffull) return 0;  // its byte offsets must stay below 2^31
-  const long nq = (p.Lq + 31) / 32, nk = (p.L + 31) / 32;
+  if (cus <= 0 || ((uint64_t)p.L + 256) * d * 2 > 0x7fffffffull) return 0;  // its byte offsets must stay below 2^31
+  const long nq = ((long)p.Lq + 31) / 32, nqb = ((long)p.Lq + 255) / 256, nb = ((long)p.L + BK - 1) / BK;
   if (nq * p.H > 0x7fffffffL / 256) return 0;
-  const long nqb = (p.Lq + 255) / 256, tiles = nqb * p.H, nb = (p.L + BK - 1) / BK;
-  double steps = (double)nq * nk * p.H, other;
+  const int di = d / 32 - 2;  // head dim 64, 96, 128: 0, 1, 2
+  const WholeTimes &w = WHOLE[di][q8];
+  const double per_cu = (double)p.H / cus;
+  double other;
   if (causal) {
-    auto keys = [&](long rows) { return std::max(0L, std::min((long)p.L, rows + p.causal_off)); };
-    steps = 0;
-    for (long t = 0; t < nq; t++) steps += (double)((keys(32 * t + 32) + 31) / 32) * p.H;
-    double total = 0;
-    for (long t = 0; t < nqb; t++) total += (double)((keys(256 * t + 256) + BK - 1) / BK) * p.H;
-    other = 5 + 2.2 * std::max((double)((keys(256 * nqb) + BK - 1) / BK), total / cus);
+    const CausalBlocks cb = causal_blocks(nqb, 256, BK, p.causal_off, p.L);
+    other = w.c_start + std::max(w.c_longest * cb.longest, (w.c_block * cb.sum + w.c_tile * nqb) * per_cu);
   } else {
-    const double start = wave ? (b16 ? 12 : 15) : d == 64 ? 3 : 5;
-    const double per = wave ? (b16 ? 1.55 : 1.8) : d == 128 ? 2.2 : d == 96 ? 1.65 : 1.5;
-    const long R = tiles % cus;
     // (the scratch memory of a split is left out: a call takes the same kernel through both entry points)
-    const long s = R ? std::min(cus / R, nb / 2) : 0;
-    const double last = R == 0 ? 0 : s >= 2 ? (double)((nb + s - 1) / s) + (wave ? 13 : 16) / per : (double)nb;
-    other = start + per * ((double)(tiles / cus) * nb + last);
+    const long tiles = nqb * p.H, full = tiles / cus, R = tiles % cus;
+    long s = R ? std::min(cus / R, nb / 2) : 0;
+    const double rows = p.Lq / (256.0 * nqb);
+    other = w.start + w.block * full * nb + w.round * full + w.rows * rows * full;
+    if (s >= 2) {
+      const long cb = (nb + s - 1) / s;
+      s = (nb + cb - 1) / cb;
+      other += w.block * cb + w.split + (w.unit_rows * rows + w.unit) * R * s + w.chunk * s;
+    } else if (R) {
+      other += w.block * nb + w.rows * rows;
+    }
   }
-  const double one = 5 + (d == 64 ? 0.5e-3 : d == 96 ? 0.7e-3 : 1.0e-3) * steps;
-  const double two = d == 96 ? 12 + 0.95e-3 * steps / 2 : 2 * one;
-  return std::min(one, two) < 0.93 * other ? (two < one ? 2 : 1) : 0;
+  auto small = [&](const SmallTimes &t, long nu) {
+    const long n = (nq + nu - 1) / nu;
+    if (causal) {
+      const CausalBlocks cb = causal_blocks(n, 32 * nu, 32, p.causal_off, p.L);
+      return t.c_start +
+             std::max(t.c_longest * std::ceil(cb.longest / 4), (t.c_block * cb.sum / 4 + t.c_tile * n) * per_cu);
+    }
+    const long wave_blocks = ((long)p.L + 127) / 128, m = (n * p.H + cus - 1) / cus, rest = m % t.slots;  // m: of a CU
+    return t.start + (m / t.slots) * (t.round + t.block[t.slots - 1] * wave_blocks) +
+           (rest ? t.round + t.block[rest - 1] * wave_blocks : 0.0);
+  };
+  const double one = small(SMALL[di][q8], 1), two = d == 96 ? small(SMALL[3][q8], 2) : one;
+  const bool pair = d == 96 && two < 0.95 * one;
+  return (pair ? two : one) < 0.95 * other ? (pair ? 2 : 1) : 0;
 }
 
 // Host side: validation (every access the kernel makes must fall inside the
@@ -637,7 +696,7 @@ int launch_attention(const Pipeline &pl, const Exec &ex, const Arg *args, int na
   }
   if (p.Lq == 0) return 0;
   if (!DUMP || usew) {
-    const int nu = pl.ival[1] ? small_tiles(D, QKT != T_I8, CAUSAL, usew, p) : 0;
+    const int nu = pl.ival[1] ? small_tiles(D, QKT == T_I8, CAUSAL, p) : 0;
     if (nu) return launch_attention_small(D, QKT, VT, OT, nu, CAUSAL, DUMP, ex, args, p, err);
   }
   const int BQ = usew ? WAVE_BQ : C::BQ;
