@@ -38,8 +38,9 @@
 // the scale and its reciprocal) is computed once for 8 rows, a row per lane;
 // the angle tables of the 8 rows are made once per workgroup in LDS, in
 // channel order, with the rotary signs and the transform's fixed signs folded
-// in; and codes are rounded by one fma each. 150 us (4.7 TB/s) there, 49 -> 44
-// us at 4608 rows; 16-bit outputs 176 -> 152 us.
+// in; and codes are rounded by one fma each. 140 us (5.0 TB/s) there, 49 -> 44
+// us at 4608 rows; 16-bit outputs 176 -> 152 us. int8 outputs without norm and
+// rotary embedding (PLAIN) take one row at a time: there is little to share.
 #include "h3hip_internal.h"
 
 #include <cmath>
@@ -118,11 +119,13 @@ __device__ __forceinline__ float group_bcast(float v, int gbase) {
 }
 
 template <int R> using RowConst = std::integral_constant<int, R>;
-// f(RowConst<0>) ... f(RowConst<RPW - 1>): the rows as compile-time constants (a DPP control has to be one)
+// f(RowConst<0>) ... f(RowConst<nr - 1>): the rows as compile-time constants (a DPP control has to be one). It ends at the
+// last row, so that a row's store is known to be behind the loads of the later rows and no wait for them waits for it
 template <class F>
-__device__ __forceinline__ void each_row(F &&f) {
-  f(RowConst<0>{}), f(RowConst<1>{}), f(RowConst<2>{}), f(RowConst<3>{});
-  f(RowConst<4>{}), f(RowConst<5>{}), f(RowConst<6>{}), f(RowConst<7>{});
+__device__ __forceinline__ void each_row(int nr, F &&f) {
+  auto go = [&](auto rc) { return decltype(rc)::value < nr && (f(rc), true); };
+  (void)(go(RowConst<0>{}) && go(RowConst<1>{}) && go(RowConst<2>{}) && go(RowConst<3>{}) && go(RowConst<4>{}) &&
+         go(RowConst<5>{}) && go(RowConst<6>{}) && go(RowConst<7>{}));
   static_assert(RPW == 8, "rows");
 }
 
@@ -134,7 +137,7 @@ __device__ __forceinline__ float flip(float v, unsigned bit) {
   return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ bit);
 }
 
-template <int HDIM, int PER, int IN_T, int QK_T, int V_T, bool QKROT>
+template <int HDIM, int PER, int IN_T, int QK_T, int V_T, bool QKROT, bool PLAIN>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restrict__ in, const float *__restrict__ wq,
                                                             const float *__restrict__ wk,
                                                             const float *__restrict__ cs,
@@ -142,6 +145,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
                                                             char *__restrict__ Ko, char *__restrict__ Vo,
                                                             float *__restrict__ qsc, float *__restrict__ ksc,
                                                             QkRopeParams p, int nd) {
+  const bool norm = !PLAIN && p.norm;  // PLAIN: int8 outputs without norm and rotary embedding (launch_qk)
+  const int rot = PLAIN ? 0 : p.rot;
   using SH = PrepassShape<HDIM, PER>;
   constexpr int LPS = SH::LPS;
   using IE = typename Elem<IN_T>::type;
@@ -154,9 +159,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
   const int l32 = lane & (LPS - 1);  // lane within the slot's group
   const int gbase = lane & ~(LPS - 1);  // first lane of the group
   const int g = group_of_lane<LPS>(l32);  // this lane's channel group: channels g * PER .. g * PER + PER - 1
-  // order of the workgroups: nd > 0 row groups of a slot group first, or -nd slot groups of a row group first (launch_qk)
-  const int nn = nd > 0 ? nd : -nd, bq = blockIdx.x / nn, br = blockIdx.x - bq * nn;
-  const int bx = nd > 0 ? br : bq, by = nd > 0 ? bq : br;
+  // order of the workgroups: the row groups of a slot group first, or the nd > 0 slot groups of a row group (launch_qk)
+  const int bx = nd ? blockIdx.x / nd : blockIdx.x, by = nd ? blockIdx.x - bx * nd : blockIdx.y;
   const int slot = by * SH::SPG + w * (64 / LPS) + lane / LPS;
   const int m0 = bx * RPW;
   const int nslots = p.Hq + p.Hk + p.Hv;
@@ -171,10 +175,10 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
 #pragma unroll
     for (int r = 0; r < RPW; r++) xin[r] = *(const IV *)(src + (size_t)min(r, nr - 1) * p.in_stride);
   }
-  const int half_rot = p.rot / 2;
-  if (p.rot && by * SH::SPG < p.Hq + p.Hk) {  // (uniform over the workgroup)
-    for (int i = threadIdx.x; i < nr * p.rot; i += 256) {
-      const int r = i / p.rot, c = i - r * p.rot;
+  const int half_rot = rot / 2;
+  if (rot && by * SH::SPG < p.Hq + p.Hk) {  // (uniform over the workgroup)
+    for (int i = threadIdx.x; i < nr * rot; i += 256) {
+      const int r = i / rot, c = i - r * rot;
       const bool first = c < half_rot;
       const size_t at = (size_t)((m0 + r) % p.seq_len) * half_rot + (first ? c : c - half_rot);
       const unsigned sb = QKROT ? sign_bit(c) : 0u;
@@ -212,15 +216,17 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
 
   // What is one value per row (the norm's 1 / sqrt, the int8 scale) is computed once for the 8 rows of a slot: lane r
   // of the group takes row r's sum (or maximum), and the result is broadcast back row by row.
-  const bool rotated = g * PER < p.rot;  // this lane's channels are in rotary pairs (they then get their signs there)
+  const bool rotated = g * PER < rot;  // this lane's channels are in rotary pairs (they then get their signs there)
   auto sign_of = [&](int i) { return QKROT && !rotated ? sign_bit(g * PER + i) : 0u; };
-  float wv[PER], inv_l = 1.0f;
-  if (p.norm) {
+  float wv[PER], inv_l = 1.0f;  // a channel's weight, with its sign
+#pragma unroll
+  for (int i = 0; i < PER; i++) wv[i] = flip(1.0f, sign_of(i));
+  if (norm) {
     const float *ws = (isq ? wq : wk) + g * PER;
 #pragma unroll
     for (int i = 0; i < PER; i++) wv[i] = flip(ws[i], sign_of(i));
     float mine = 1.0f;
-    each_row([&](auto rc) {
+    each_row(RPW, [&](auto rc) {
       constexpr int r = decltype(rc)::value;
       float ss = (float)xin[r][0] * (float)xin[r][0];
 #pragma unroll
@@ -241,15 +247,15 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
   // row r normalised and rotated (and, on QKROT, with its signs)
   auto row = [&](auto rc, float (&v)[PER]) __attribute__((always_inline)) {
     constexpr int r = decltype(rc)::value;
-    if (p.norm) {
+    if (norm) {
       const float inv = group_bcast<LPS, r>(inv_l, gbase);
 #pragma unroll
       for (int i = 0; i < PER; i++) v[i] = ((float)xin[r][i] * inv) * wv[i];
     } else {
 #pragma unroll
-      for (int i = 0; i < PER; i++) v[i] = flip((float)xin[r][i], sign_of(i));
+      for (int i = 0; i < PER; i++) v[i] = (float)xin[r][i] * wv[i];
     }
-    if (p.rot) {
+    if (rot) {
       float pv[PER];
 #pragma unroll
       for (int i = 0; i < PER; i++)
@@ -267,9 +273,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
   if constexpr (QK_T != T_I8) {
     using OE = typename Elem<QK_T>::type;
     typedef typename VecOf<PER, OE>::type OV;
-    each_row([&](auto rc) {
+    each_row(nr, [&](auto rc) {
       constexpr int r = decltype(rc)::value;
-      if (r >= nr) return;
       float v[PER];
       row(rc, v);
       OV out;
@@ -281,19 +286,18 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
     // the transform's final factor 1 / sqrt(HDIM), with the sign that the lane carries (an exact sign change)
     constexpr float rn = QKROT ? (float)inv_sqrt_hdim<HDIM>() : 1.0f;
     const float rns = QKROT && (__builtin_popcount(g) & 1) ? -rn : rn;
-    float v[RPW][PER], mine = 0.0f;
-    each_row([&](auto rc) {
-      constexpr int r = decltype(rc)::value;
-      row(rc, v[r]);
+    // a row normalised, rotated and transformed, but for that factor, and the largest magnitude of its values
+    auto transform = [&](auto rc, float (&v)[PER]) __attribute__((always_inline)) {
+      row(rc, v);
       if constexpr (QKROT) {
 #pragma unroll
         for (int s = 1; s < PER; s <<= 1) {
 #pragma unroll
           for (int i = 0; i < PER; i++) {
             if (!(i & s)) {
-              const float a = v[r][i], b = v[r][i + s];
-              v[r][i] = a + b;
-              v[r][i + s] = a - b;
+              const float a = v[i], b = v[i + s];
+              v[i] = a + b;
+              v[i + s] = a - b;
             }
           }
         }
@@ -302,7 +306,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
         // times (-1)^popcount(g) (hadamard_lane_stage)
         auto stage = [&](auto ls_const) {
           constexpr int LS = decltype(ls_const)::value;
-          group_stage<LPS, LS>(v[r], (g & LS) ? -1.0f : 1.0f);
+          group_stage<LPS, LS>(v, (g & LS) ? -1.0f : 1.0f);
         };
         stage(std::integral_constant<int, 1>{});
         stage(std::integral_constant<int, 2>{});
@@ -312,48 +316,73 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const char *__restric
       }
       float amax = 0.0f;
 #pragma unroll
-      for (int i = 0; i < PER; i++) amax = fmaxf(amax, fabsf(v[r][i]));
+      for (int i = 0; i < PER; i++) amax = fmaxf(amax, fabsf(v[i]));
       if constexpr (LPS > 16) amax = fmaxf(amax, gshfl<LPS, 16>(amax));
       if constexpr (LPS > 8) amax = fmaxf(amax, gshfl<LPS, 8>(amax));
       amax = fmaxf(amax, gshfl<LPS, 4>(amax));
       amax = fmaxf(amax, gshfl<LPS, 2>(amax));
-      amax = fmaxf(amax, gshfl<LPS, 1>(amax));
-      if (l32 == r) mine = amax;
-    });
+      return fmaxf(amax, gshfl<LPS, 1>(amax));
+    };
     // rounding is monotonic, so the largest |v * rn| is the rounded product of the largest |v|
-    const float am = QKROT ? mine * rn : mine;
-    const float scale_l = am > 0.0f ? am / 127.0f : 1.0f;
-    const float rs_l = __builtin_amdgcn_rcpf(scale_l);  // 1 ulp
-    each_row([&](auto rc) {
+    auto scale_of = [&](float amax) {
+      const float am = QKROT ? amax * rn : amax;
+      return am > 0.0f ? am / 127.0f : 1.0f;
+    };
+    // Codes are the nearest integers of fl(v * rns) / scale. y = v * (rns * rs) is within 2^-14 of that quotient
+    // (|y| <= 128; four roundings of at most 1 ulp), so their nearest integers agree unless y lies within 2^-14 of
+    // a half-integer, and then the wave divides (one row of four slots in sixteen, and exact). t = fma(v, f, 1.5 * 2^23)
+    // rounds y to the nearest integer (half to even), whose two's complement is in t's low bits. A scale whose
+    // reciprocal (rs, 1 ulp) is not a normal float (amax below ~2^-119) divides too, and so does a NaN (`far` keeps it).
+    auto code = [&](auto rc, const float (&v)[PER], float rs, auto scale) __attribute__((always_inline)) {
       constexpr int r = decltype(rc)::value;
-      if (r >= nr) return;
-      // Codes are the nearest integers of fl(v * rns) / scale. y = v * (rns * rs) is within 2^-14 of that quotient
-      // (|y| <= 128; four roundings of at most 1 ulp), so their nearest integers agree unless y lies within 2^-14 of
-      // a half-integer, and then the wave divides (one row of four slots in sixteen, and exact). t = fma(v, f, 1.5 * 2^23) rounds y to
-      // the nearest integer (half to even), whose two's complement is in t's low bits. A scale whose reciprocal is not
-      // a normal float (amax below ~2^-119) divides too, and so does a NaN (`far` keeps it).
-      const float rs = group_bcast<LPS, r>(rs_l, gbase), f = rs * rns;
+      const float f = rs * rns;
       constexpr float MG = 12582912.0f;
       unsigned t[PER];
       float far = 0.0f;
 #pragma unroll
       for (int i = 0; i < PER; i++) {
-        const float ti = __builtin_fmaf(v[r][i], f, MG);
-        far = __builtin_elementwise_maximum(far, fabsf(__builtin_fmaf(v[r][i], f, -(ti - MG))));
+        const float ti = __builtin_fmaf(v[i], f, MG);
+        far = __builtin_elementwise_maximum(far, fabsf(__builtin_fmaf(v[i], f, -(ti - MG))));
         t[i] = __builtin_bit_cast(unsigned, ti);
       }
-      // wave-uniform, so that the broadcast's source lanes are active
-      if (__builtin_amdgcn_ballot_w64(!(far <= 0.5f - 0x1p-14f) || !(rs < 0x1p126f))) {
-        const float scale = group_bcast<LPS, r>(scale_l, gbase);
+      bool divide = !(far <= 0.5f - 0x1p-14f) || !(rs < 0x1p126f);
+      if constexpr (!PLAIN) divide = __builtin_amdgcn_ballot_w64(divide);  // so that a broadcast's source lanes are active
+      if (divide) {
+        const float s = scale(rc);
 #pragma unroll
-        for (int i = 0; i < PER; i++) t[i] = (unsigned)(int)rintf((QKROT ? v[r][i] * rns : v[r][i]) / scale);
+        for (int i = 0; i < PER; i++) t[i] = (unsigned)(int)rintf((QKROT ? v[i] * rns : v[i]) / s);
       }
       typedef typename VecOf<PER, signed char>::type CV;
       CV codes;
 #pragma unroll
       for (int i = 0; i < PER; i++) codes[i] = (signed char)t[i];
       st((CV *)((isq ? Qo : Ko) + hrow_of(m0 + r) * HDIM + g * PER), codes);
-    });
+    };
+    float scale_l = 1.0f;  // of row l32
+    if constexpr (PLAIN) {
+      // one row at a time
+      each_row(nr, [&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        float v[PER];
+        const float scale = scale_of(transform(rc, v));
+        code(rc, v, __builtin_amdgcn_rcpf(scale), [&](auto) { return scale; });
+        if (l32 == r) scale_l = scale;
+      });
+    } else {
+      float v[RPW][PER], mine = 0.0f;
+      each_row(RPW, [&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        const float amax = transform(rc, v[r]);
+        if (l32 == r) mine = amax;
+      });
+      scale_l = scale_of(mine);
+      const float rs_l = __builtin_amdgcn_rcpf(scale_l);
+      each_row(nr, [&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        code(rc, v[r], group_bcast<LPS, r>(rs_l, gbase),
+             [&](auto q) { return group_bcast<LPS, decltype(q)::value>(scale_l, gbase); });
+      });
+    }
     if (l32 < nr) (isq ? qsc : ksc)[hrow_of(m0 + l32)] = scale_l;
   }
 }
@@ -434,24 +463,38 @@ int launch_qk(const Pipeline &pl, const Exec &ex, const Arg *a, int nargs, const
   if (p.M == 0) return 0;
   // 8 channels per lane (16-byte loads for 16-bit inputs) unless the rotary pairs would straddle lanes, then
   // the reference's HDIM / 32
-  auto go = [&](auto per_const) {
+  auto go = [&](auto per_const, auto plain) {
     constexpr int P = decltype(per_const)::value;
     constexpr int SPG = PrepassShape<HDIM, P>::SPG;
     const int nx = (p.M + RPW - 1) / RPW, ny = (nslots + SPG - 1) / SPG;
-    const dim3 grid((unsigned)nx * ny);
-    // The order of the workgroups. int8 calls whose rows outgrow the 256 MB last-level cache together with the outputs
-    // run a row group's slot groups first, so that the value copies overlap the queries' and keys' arithmetic (415 MB
-    // of rows: 171 -> 153 us, 201 MB: 82 -> 76). Otherwise the row groups of a slot group's 4 KB columns go first
-    // (113 MB of rows just written by a projection: 50 -> 45 us, 37 MB: 23 -> 20; 16-bit outputs 31 -> 29 at 85 MB).
-    const bool rows_first = QK_T == T_I8 && (uint64_t)p.M * nslots * HDIM * esize(IN_T) > 160000000ull;
-    hipLaunchKernelGGL((qk_norm_rope_kernel<HDIM, P, IN_T, QK_T, V_T, QKROT>), grid, dim3(256), 0, ex.stream, a[0].ptr,
+    // The order of the workgroups. int8 calls with a rotary embedding whose 16-bit rows outgrow the 256 MB last-level
+    // cache together with the outputs run a row group's slot groups first, so that the value copies overlap the queries'
+    // and keys' arithmetic (415 MB of rows: 153 -> 139 us, 221 MB: 72 -> 69). Otherwise the row groups of a slot group's
+    // columns go first (113 MB of rows just written by a projection: 50 -> 45 us; 415 MB without norm and embedding: 138
+    // -> 130; float32 rows, 207 MB: 56 -> 45).
+    const bool rows_first = QK_T == T_I8 && IN_T != T_F32 && p.rot &&
+                            (uint64_t)p.M * nslots * HDIM * esize(IN_T) > 160000000ull;
+    // PLAIN is bound by HBM, and its 54 to 96 registers would let 5 to 8 waves run on a SIMD: an unused LDS request holds it
+    // to 5 (4 with float32 rows), whose accesses lie closer together (415 MB of rows without the transform: 130 -> 125 us)
+    const unsigned lds = !decltype(plain)::value ? 0 : IN_T == T_F32 ? 40000 : 32000;
+    const dim3 grid = rows_first ? dim3((unsigned)nx * ny) : dim3((unsigned)nx, (unsigned)ny);
+    hipLaunchKernelGGL((qk_norm_rope_kernel<HDIM, P, IN_T, QK_T, V_T, QKROT, decltype(plain)::value>), grid, dim3(256), lds, ex.stream, a[0].ptr,
                        (const float *)a[1].ptr, (const float *)a[2].ptr, (const float *)a[3].ptr,
                        (const float *)a[4].ptr, a[5].ptr, a[6].ptr, a[7].ptr,
                        nargs > 9 ? (float *)a[9].ptr : nullptr, nargs > 10 ? (float *)a[10].ptr : nullptr, p,
-                       rows_first ? -ny : nx);
+                       rows_first ? ny : 0);
   };
-  if ((p.rot / 2) % 8 == 0) go(std::integral_constant<int, 8>{});
-  else go(std::integral_constant<int, HDIM / 32>{});
+  if constexpr (QK_T == T_I8) {
+    // PLAIN: what is one value per row is little here, and holding 8 rows' values for it took 126 registers (with the order
+    // and the occupancy above 10.1 -> 9.1 us at 1000 rows of 32 + 32 + 32 heads, 35.0 -> 31.1 at 4608; without the transform
+    // 133 -> 125 at 16896)
+    if (!p.norm && !p.rot) {
+      go(std::integral_constant<int, 8>{}, std::true_type{});
+      return 0;
+    }
+  }
+  if ((p.rot / 2) % 8 == 0) go(std::integral_constant<int, 8>{}, std::false_type{});
+  else go(std::integral_constant<int, HDIM / 32>{}, std::false_type{});
   return 0;
 }
 

@@ -337,3 +337,32 @@ def test_codes_at_half_integers(gpu, hd):
     want = op.qk_norm_rope(x, Hq=H, Hk=H, Hv=H, hd=hd, out_rows=64, rot=0, eps=1e-6, norm=False, q8=True, qk_rot=False)
     for n in ("Q", "K", "qs", "ks"):
         assert np.array_equal(got[n][:, :M], want[n][:, :M]), n
+
+
+@pytest.mark.parametrize("in_dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("M,Hq,Hk,Hv", [(1, 1, 1, 1), (7, 5, 2, 9), (8, 16, 16, 16), (9, 33, 31, 1)])
+def test_int8_rows_one_at_a_time(gpu, in_dt, hd, M, Hq, Hk, Hv):
+    """int8 outputs without norm and rotary embedding, whose kernel takes one row at a time: row counts around its 8
+    rows, head counts that leave queries, keys and values in one wave and lane groups without a head; with a row of
+    zeros and a head with a NaN (code 0; the scale of its finite values, 1 behind the rotation). Codes and scales bit for
+    bit, with the rotation and without."""
+    rng = np.random.default_rng(M * hd + Hq)
+    S = Hq + Hk + Hv
+    x = outlier_rows(rng, M, S, hd)[:, :S * hd]
+    x[M // 2, :hd * Hq] = 0
+    xh = to_bf16(x) if in_dt == "bf16" else x.astype(np.float16 if in_dt == "f16" else np.float32)
+    xh[M - 1, Hq * hd + 3] = {"bf16": np.uint16(0x7FC0)}.get(in_dt, np.nan)  # the first key head
+    for qk_rot in (True, False):
+        got = run_prepass(gpu, xh, in_dt, M=M, Hq=Hq, Hk=Hk, Hv=Hv, hd=hd, out_rows=16, qk_rot=qk_rot)
+        xf = as_float(xh, in_dt).copy()
+        xf[M - 1, Hq * hd + 3] = 0
+        if qk_rot:
+            xf[M - 1, Hq * hd:(Hq + 1) * hd] = 0
+        want = op.qk_norm_rope(xf, Hq=Hq, Hk=Hk, Hv=Hv, hd=hd, out_rows=16, rot=0, eps=1e-6, norm=False, q8=True,
+                               qk_rot=qk_rot)
+        for n in ("Q", "K"):
+            assert np.array_equal(got[n][:, :M], want[n][:, :M]), n
+        for n in ("qs", "ks"):
+            assert np.array_equal(got[n][:, :M].view(np.uint32), want[n][:, :M].view(np.uint32)), n
+        assert np.array_equal(got["V"][:, :M].view(np.uint16), to_bf16(want["V"][:, :M]))
