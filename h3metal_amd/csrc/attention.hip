@@ -553,6 +553,11 @@ CausalBlocks causal_blocks(long n, long rows, long blk, long off, long L) {
   return {sum, (double)std::max(0L, std::min(top, k * n + c))};
 }
 
+// Whether the small tiles can run a call: their byte offsets must stay below 2^31, and their grid
+bool small_fits(int d, const AttnParams &p) {
+  return ((uint64_t)p.L + 256) * d * 2 <= 0x7fffffffull && ((long)p.Lq + 31) / 32 * p.H <= 0x7fffffffL / 256;
+}
+
 // Whether a call runs on the small tiles: 0 no, else the 32-row query tiles per workgroup (1, or 2 at head dim 96). They
 // have to be estimated 5% faster than the 256-row tiles, and two query tiles 5% faster than one. Over the calls above the
 // choice costs 0.4% on average against the best kernel of each (1.39x at worst), and 7 of them are over 5% slower than on
@@ -562,9 +567,8 @@ CausalBlocks causal_blocks(long n, long rows, long blk, long off, long L) {
 // 24.0 -> 11.4, head dim 96 H 16 1037 rows 31.9 -> 20.5, head dim 64 H 128 200 rows 24.4 -> 8.5.
 int small_tiles(int d, bool q8, bool causal, const AttnParams &p) {
   const long cus = cu_count();
-  if (cus <= 0 || ((uint64_t)p.L + 256) * d * 2 > 0x7fffffffull) return 0;  // its byte offsets must stay below 2^31
+  if (cus <= 0 || !small_fits(d, p)) return 0;
   const long nq = ((long)p.Lq + 31) / 32, nqb = ((long)p.Lq + 255) / 256, nb = ((long)p.L + BK - 1) / BK;
-  if (nq * p.H > 0x7fffffffL / 256) return 0;
   const int di = d / 32 - 2;  // head dim 64, 96, 128: 0, 1, 2
   const WholeTimes &w = WHOLE[di][q8];
   const double per_cu = (double)p.H / cus;
@@ -696,7 +700,12 @@ int launch_attention(const Pipeline &pl, const Exec &ex, const Arg *args, int na
   }
   if (p.Lq == 0) return 0;
   if (!DUMP || usew) {
-    const int nu = pl.ival[1] ? small_tiles(D, QKT == T_I8, CAUSAL, p) : 0;
+    const int nu = pl.ival[1] < 0 ? small_tiles(D, QKT == T_I8, CAUSAL, p) : pl.ival[1];
+    if (pl.ival[1] > 0 && !small_fits(D, p)) {
+      *err = "Lq " + std::to_string(p.Lq) + ", L " + std::to_string(p.L) + ", H " + std::to_string(p.H) +
+             ": too large for the small tiles (SMALL)";
+      return -1;
+    }
     if (nu) return launch_attention_small(D, QKT, VT, OT, nu, CAUSAL, DUMP, ex, args, p, err);
   }
   const int BQ = usew ? WAVE_BQ : C::BQ;
@@ -795,7 +804,8 @@ int type_of(const std::string &s) {
 // SPLIT=0 runs every tile whole. GROUPS (this build's): 1 the wave-pipelined
 // kernel for HD 128 without a causal mask at every size, 0 (the default) the
 // small tiles where they are faster (the values that selected other kernels are
-// refused).
+// refused). SMALL (this build's) names the small tiles at every size, whichever
+// is faster: their 32-row query tiles per workgroup, 1, or 2 with HD 96.
 bool make_attention(const std::string &fn, const Macros &m, Pipeline *pl, std::string *err) {
   const bool dump = fn == "attention_scores";
   if (fn != "attention" && !dump) {
@@ -808,8 +818,10 @@ bool make_attention(const std::string &fn, const Macros &m, Pipeline *pl, std::s
     return false;
   for (const char *k : {"WM", "BK", "KPAD", "DB", "PVORDER", "VX", "SLACK", "TG"})
     if (!macro_int(m, k, 0, &dummy, err)) return false;
-  int split, groups;
-  if (!macro_int(m, "SPLIT", 1, &split, err) || !macro_int(m, "GROUPS", 0, &groups, err)) return false;
+  int split, groups, small;
+  if (!macro_int(m, "SPLIT", 1, &split, err) || !macro_int(m, "GROUPS", 0, &groups, err) ||
+      !macro_int(m, "SMALL", 0, &small, err))
+    return false;
   if (groups < 0 || groups > 1) {
     *err = "GROUPS must be 0 or 1 (the wave-pipelined kernel; the paired, ping-pong and two-group kernels that 2-4 "
            "selected for HD 128 without a causal mask are retired)";
@@ -817,7 +829,7 @@ bool make_attention(const std::string &fn, const Macros &m, Pipeline *pl, std::s
   }
   for (auto &kv : m) {
     static const char *known[] = {"HD", "QK8", "CAUSAL", "O_T", "IN_T", "WM", "BK", "KPAD", "DB", "PVORDER", "VX",
-                                  "SLACK", "TG", "SPLIT", "GROUPS"};
+                                  "SLACK", "TG", "SPLIT", "GROUPS", "SMALL"};
     bool ok = false;
     for (const char *k : known) ok = ok || kv.first == k;
     if (!ok) {
@@ -835,6 +847,12 @@ bool make_attention(const std::string &fn, const Macros &m, Pipeline *pl, std::s
     *err = "HD " + std::to_string(hd) + " not supported (64, 96 or 128)";
     return false;
   }
+  const bool wave = hd == 128 && !causal;
+  if (small < 0 || small > (hd == 96 ? 2 : 1) || (small && (!split || groups || (dump && !wave)))) {
+    *err = "SMALL must be 0, 1, or 2 with HD 96; not with SPLIT=0, GROUPS=1, or the scores hook of other than HD 128 "
+           "without a causal mask";
+    return false;
+  }
   const int qkt = qk8 ? T_I8 : it;
   LaunchFn f;
   if (hd == 128) f = dump ? pick_types<128, true>(qkt, it, ot, causal) : pick_types<128, false>(qkt, it, ot, causal);
@@ -843,10 +861,11 @@ bool make_attention(const std::string &fn, const Macros &m, Pipeline *pl, std::s
   pl->launch = f;
   // the kernel the pipeline launches: 1 the wave-pipelined kernel (HD 128 without a causal mask), 0 this file's
   // two-group kernel (every other case)
-  const int ksel = hd == 128 && !causal ? 1 : 0;
+  const int ksel = wave ? 1 : 0;
   pl->threads = ksel == 1 ? WAVE_THREADS : NW * 64;
   pl->ival[0] = split != 0;
-  pl->ival[1] = split != 0 && groups == 0;  // the small tiles split the keys, and GROUPS=1 names a kernel
+  // the small tiles: named, chosen by the size (-1), or not taken (they split the keys, and GROUPS=1 names a kernel)
+  pl->ival[1] = small ? small : split != 0 && groups == 0 ? -1 : 0;
   pl->ival[2] = ksel;
   return true;
 }

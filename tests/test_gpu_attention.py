@@ -19,6 +19,8 @@ from oracle.bf16 import from_bf16, to_bf16
 pytestmark = pytest.mark.gpu
 
 NS_MAX, NS_MEAN = 2e-2, 1e-3
+# what runs a call at D = 128 without a causal mask: the wave-pipelined kernel, or the small tiles
+KERNELS = pytest.mark.parametrize("kernel", [dict(GROUPS=1), dict(SMALL=1)], ids=["wave", "small"])
 
 
 def q8(x):
@@ -60,9 +62,12 @@ def run_attention(gpu, q, k, v, *, dtype, Lq, L, H, KVH, D, scale, causal=False,
 
 @pytest.mark.parametrize("Lq,L,H,KVH,D", [(100, 100, 2, 2, 128), (77, 300, 3, 3, 128), (64, 64, 4, 1, 64),
                                           (300, 1037, 2, 1, 128), (1, 5, 1, 1, 128), (700, 449, 2, 2, 128)])
-def test_int32_scores_bit_exact(gpu, Lq, L, H, KVH, D):
-    """int32 score accumulators of the kernel that runs equal the exact integer products (int8: D=128 the
-    wave-pipelined kernel, D=64 the two-group one)."""
+@KERNELS
+def test_int32_scores_bit_exact(gpu, kernel, Lq, L, H, KVH, D):
+    """int32 score accumulators equal the exact integer products: at D=128 those of the wave-pipelined kernel and of
+    the small tiles, at D=64 those of the two-group kernel (the scores hook has no small tiles there)."""
+    if D != 128:
+        kernel = {"GROUPS": kernel.get("GROUPS", 0)}
     rng = np.random.default_rng(Lq + L)
     qi = rng.integers(-127, 128, (H, Lq, D)).astype(np.int8)
     ki = rng.integers(-127, 128, (KVH, L, D)).astype(np.int8)
@@ -75,14 +80,15 @@ def test_int32_scores_bit_exact(gpu, Lq, L, H, KVH, D):
     S = gpu.empty((H, Lq, L), "i32")
     print(f"[scores] Lq={Lq} L={L} H={H} KVH={KVH} D={D}", flush=True)
     ops.attention_scores(gpu, Q, K, V, S, Lq=Lq, L=L, H=H, KVH=KVH, D=D, q_rows=q_rows, k_rows=k_rows,
-                         q_scale=qs, k_scale=ks)
+                         q_scale=qs, k_scale=ks, **kernel)
     gpu.wait()
     want = oa.int_scores(qi, ki, H_per_kv=H // KVH)
     got = S.numpy()
     assert np.array_equal(got, want), f"{(got != want).sum()} int32 scores differ"
 
 
-def test_int32_scores_golden_fixture(gpu):
+@KERNELS
+def test_int32_scores_golden_fixture(gpu, kernel):
     import os
     f = np.load(os.path.join(os.path.dirname(__file__), "golden", "scores_int8.npz"))
     qi, ki, want = f["Q"], f["K"], f["S"]
@@ -92,13 +98,14 @@ def test_int32_scores_golden_fixture(gpu):
     S = gpu.empty((H, Lq, L), "i32")
     ops.attention_scores(gpu, Q, K, gpu.empty((H, 64, D), "bf16"), S, Lq=Lq, L=L, H=H, KVH=H, D=D, q_rows=64,
                          k_rows=64, q_scale=gpu.upload(np.ones((H, 64), np.float32)),
-                         k_scale=gpu.upload(np.ones((H, 64), np.float32)))
+                         k_scale=gpu.upload(np.ones((H, 64), np.float32)), **kernel)
     gpu.wait()
     assert np.array_equal(S.numpy(), want)
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
-def test_float_scores(gpu, dtype):
+@KERNELS
+def test_float_scores(gpu, kernel, dtype):
     """16-bit inputs: products are exact in fp32 and the 128-term sums are accumulated in fp32."""
     rng = np.random.default_rng(5)
     H, Lq, L, D = 2, 70, 130, 128
@@ -112,7 +119,7 @@ def test_float_scores(gpu, dtype):
     Q, K = padded(gpu, qh, 128, dtype), padded(gpu, kh, 160, dtype)
     S = gpu.empty((H, Lq, L), "f32")
     ops.attention_scores(gpu, Q, K, gpu.empty((H, 160, D), dtype), S, Lq=Lq, L=L, H=H, KVH=H, D=D, q_rows=128,
-                         k_rows=160)
+                         k_rows=160, **kernel)
     gpu.wait()
     want = np.einsum("hqd,hkd->hqk", qf.astype(np.float64), kf.astype(np.float64))
     np.testing.assert_allclose(S.numpy(), want, rtol=0, atol=1e-3)
@@ -289,9 +296,10 @@ def test_config3_zimage_key_padding(gpu):
     assert err.max() < NS_MAX and err.mean() < NS_MEAN, (err.max(), err.mean(), L_txt)
 
 
-def test_config4_int32_scores_and_output_at_full_key_length(gpu):
-    """The config-4 key count (L = 16896) through the scores hook, which runs ops.attention's own kernel
-    (same tiles, LDS staging, tail split of the last round of tiles, P V and output): int32 scores of every
+@KERNELS
+def test_config4_int32_scores_and_output_at_full_key_length(gpu, kernel):
+    """The config-4 key count (L = 16896) through the scores hook, which runs ops.attention's own kernels (the same
+    tiles, LDS staging, P V and output; the wave-pipelined one with its tail split): int32 scores of every
     (query, key) pair of two heads bit-exact against exact integer products, and the output of the same launch
     against float64 attention of the dequantised inputs."""
     rng = np.random.default_rng(44)
@@ -309,9 +317,9 @@ def test_config4_int32_scores_and_output_at_full_key_length(gpu):
     qs, ks = gpu.upload(qsc), gpu.upload(ksc)
     S = gpu.empty((H, Lq, L), "i32")
     O = gpu.empty((Lq, H * D), "bf16")
-    print(f"[scores] full key length Lq={Lq} L={L} H={H} (split last round)", flush=True)
+    print(f"[scores] full key length Lq={Lq} L={L} H={H} {kernel}", flush=True)
     ops.attention_scores(gpu, Q, K, V, S, Lq=Lq, L=L, H=H, KVH=H, D=D, q_rows=Lq, k_rows=L, q_scale=qs,
-                         k_scale=ks, out=O, scale=D ** -0.5)
+                         k_scale=ks, out=O, scale=D ** -0.5, **kernel)
     gpu.wait()
     want = oa.int_scores(qi, ki)
     got = S.numpy()
@@ -323,7 +331,7 @@ def test_config4_int32_scores_and_output_at_full_key_length(gpu):
 
 
 def test_int32_scores_and_output_in_reversed_rounds(gpu):
-    """Enough workgroups that every other round of an XCD's workgroups takes its key blocks in the order
+    """The wave-pipelined kernel with enough workgroups that every other round of an XCD's workgroups takes its key blocks in the order
     L-2, ..., 0, L-1 (520 one-tile heads: the rounds after the first 256 workgroups run reversed), with a ragged
     last block (L = 300: 5 blocks, the last with 44 keys) and GQA (8 key/value heads): the int32 scores of every
     head bit-exact against exact integer products (the scores hook writes each at its key index, so a block
@@ -341,7 +349,7 @@ def test_int32_scores_and_output_in_reversed_rounds(gpu):
     O = gpu.empty((Lq, H * D), "bf16")
     print(f"[scores] reversed rounds H={H} KVH={KVH} Lq={Lq} L={L}", flush=True)
     ops.attention_scores(gpu, Q, K, V, S, Lq=Lq, L=L, H=H, KVH=KVH, D=D, q_rows=Lq, k_rows=L, q_scale=qs,
-                         k_scale=ks, out=O, scale=D ** -0.5)
+                         k_scale=ks, out=O, scale=D ** -0.5, GROUPS=1)
     gpu.wait()
     g = H // KVH
     kf = ki.astype(np.float64)
@@ -529,45 +537,50 @@ def test_te_n_valid_split_dispatch(gpu):
     assert (got[T:] == 0).all()
 
 
-@pytest.mark.parametrize("q8_path", [False, True])
-def test_tail_split_matches_whole_tiles(gpu, q8_path):
-    """The last, partly filled round of workgroups is cut along the keys and merged (online-softmax merge of
-    per-chunk O, m, l). Same inputs with SPLIT=0 (every tile whole): outputs agree to rounding, and both meet
-    the tolerance against float64. Here 2 heads x 2 query blocks = 4 tiles on 256 CUs: every tile is split."""
+@pytest.mark.parametrize("path", ["bf16", "f16", "int8"])
+@pytest.mark.parametrize("D", [128, 96, 64])
+def test_tail_split_matches_whole_tiles(gpu, path, D):
+    """The last, partly filled round of 256-row tiles (GROUPS=1) is cut along the keys and merged (online-softmax merge
+    of per-chunk O, m, l). Same inputs with SPLIT=0 (every tile whole): outputs agree to rounding but are not the same
+    bits (so there was a split), and both meet the tolerance against float64. Here 2 heads x 2 query blocks = 4 tiles
+    on 256 CUs: every tile is split. D=128: the wave-pipelined kernel, 96 and 64: the two-group one."""
     rng = np.random.default_rng(35)
-    H, Lq, L, D = 2, 300, 1037, 128
-    if q8_path:
+    H, Lq, L = 2, 300, 1037
+    vt = "f16" if path == "f16" else "bf16"
+    bits = (lambda x: x.astype(np.float16)) if vt == "f16" else to_bf16
+    val = (lambda x: x.astype(np.float64)) if vt == "f16" else from_bf16
+    if path == "int8":
         qi, qs = q8(rng.standard_normal((H, Lq, D)).astype(np.float32))
         ki, ks = q8(rng.standard_normal((H, L, D)).astype(np.float32))
         q, k, extra = qi, ki, dict(q_scale=padded(gpu, qs, 512, "f32"), k_scale=padded(gpu, ks, 1056, "f32"))
         qdt, ref_q, ref_k = "i8", qi * qs[..., None].astype(np.float64), ki * ks[..., None].astype(np.float64)
     else:
-        q = to_bf16(rng.standard_normal((H, Lq, D)).astype(np.float32))
-        k = to_bf16(rng.standard_normal((H, L, D)).astype(np.float32))
-        extra, qdt, ref_q, ref_k = {}, "bf16", from_bf16(q), from_bf16(k)
-    v = to_bf16(rng.standard_normal((H, L, D)).astype(np.float32))
-    Q, K, V = padded(gpu, q, 512, qdt), padded(gpu, k, 1056, qdt), padded(gpu, v, 1056, "bf16")
+        q = bits(rng.standard_normal((H, Lq, D)).astype(np.float32))
+        k = bits(rng.standard_normal((H, L, D)).astype(np.float32))
+        extra, qdt, ref_q, ref_k = {}, vt, val(q), val(k)
+    v = bits(rng.standard_normal((H, L, D)).astype(np.float32))
+    Q, K, V = padded(gpu, q, 512, qdt), padded(gpu, k, 1056, qdt), padded(gpu, v, 1056, vt)
     outs = []
     for split in (1, 0):
+        print(f"[attention] split={split} {path} D={D}", flush=True)
         O = gpu.empty((512, H * D), "f32")
         ops.attention(gpu, Q, K, V, O, Lq=Lq, L=L, H=H, KVH=H, D=D, q_rows=512, k_rows=1056, scale=D ** -0.5,
-                      SPLIT=split, **extra)
+                      SPLIT=split, GROUPS=1, **extra)
         gpu.wait()
         outs.append(O.numpy().astype(np.float64))
-    ref = oa.ref_attention(ref_q, ref_k, from_bf16(v), D ** -0.5)
+    ref = oa.ref_attention(ref_q, ref_k, val(v), D ** -0.5)
     for o in outs:
         err = np.abs(o[:Lq] - ref)
         assert err.max() < NS_MAX and err.mean() < NS_MEAN, (err.max(), err.mean())
-    assert np.abs(outs[0] - outs[1]).max() < 2e-3
+    assert 0 < np.abs(outs[0] - outs[1]).max() < 2e-3
     assert (outs[0][Lq:] == 0).all()
 
 
 @pytest.mark.parametrize("H,KVH,Lq,L,seq", [(4, 4, 1000, 1500, None), (6, 2, 777, 2049, None), (4, 4, 300, 700, 2)])
 def test_int8_split_and_whole_tiles_agree(gpu, H, KVH, Lq, L, seq):
-    """int8 scores at D=128 without a causal mask (the wave-pipelined kernel), the default GROUPS=0 and the
-    explicit GROUPS=1, with the tail split and without (SPLIT=0). Same inputs through all,
-    with and without the tail split: every output meets the tolerance against float64 and the kernels agree to
-    rounding. Ragged L (a partly masked last key block), GQA, several 256-row query blocks per head and batched
+    """int8 scores at D=128 without a causal mask: the default (GROUPS=0), the small tiles, and the wave-pipelined kernel
+    (GROUPS=1) with the tail split and without (SPLIT=0). Same inputs through all: every output meets the tolerance
+    against float64 and the kernels agree to rounding. Ragged L (a partly masked last key block), GQA, several 256-row query blocks per head and batched
     sequences (seq_heads) included."""
     rng = np.random.default_rng(H * 1000 + L)
     D = 128
@@ -580,11 +593,11 @@ def test_int8_split_and_whole_tiles_agree(gpu, H, KVH, Lq, L, seq):
     seq_heads = seq or H
     nseq = H // seq_heads
     outs = []
-    for groups, split in ((0, 1), (1, 1), (1, 0)):
-        print(f"[attention] groups={groups} split={split} H={H} KVH={KVH} Lq={Lq} L={L} seq={seq}", flush=True)
+    for kernel in (dict(GROUPS=0), dict(SMALL=1), dict(GROUPS=1), dict(GROUPS=1, SPLIT=0)):
+        print(f"[attention] {kernel} H={H} KVH={KVH} Lq={Lq} L={L} seq={seq}", flush=True)
         O = gpu.empty((nseq * qr, seq_heads * D), "f32")
         ops.attention(gpu, Q, K, V, O, Lq=Lq, L=L, H=H, KVH=KVH, D=D, q_rows=qr, k_rows=kr, scale=D ** -0.5,
-                      seq_heads=seq_heads, seq_rows=qr, GROUPS=groups, SPLIT=split, **extra)
+                      seq_heads=seq_heads, seq_rows=qr, **kernel, **extra)
         gpu.wait()
         outs.append(O.numpy().astype(np.float64))
     rq = qi * qs[..., None].astype(np.float64)
@@ -609,8 +622,9 @@ def test_groups_macro_refused(gpu):
 
 @pytest.mark.parametrize("Lq,L", [(1, 1), (5, 63), (384, 64), (385, 65), (17, 129), (700, 191), (64, 31), (65, 33),
                                   (257, 97), (200, 160)])
-def test_int8_kernel_edges(gpu, Lq, L):
-    """Edge shapes through the wave-pipelined kernel (int8, D=128, no causal mask): one query or one key, key counts
+@KERNELS
+def test_int8_kernel_edges(gpu, kernel, Lq, L):
+    """Edge shapes through the wave-pipelined kernel and the small tiles (int8, D=128, no causal mask): one query or one key, key counts
     around the 64-key block and its 32-key tiles
     (the last block's rows past L load as zeros and are masked), query counts around the 64-row pairs and the
     256-row tiles. Checked against float64 within the north-star tolerance."""
@@ -624,7 +638,7 @@ def test_int8_kernel_edges(gpu, Lq, L):
     O = gpu.empty((qr, H * D), "f32")
     print(f"[attention] edge Lq={Lq} L={L}", flush=True)
     ops.attention(gpu, Q, K, V, O, Lq=Lq, L=L, H=H, KVH=H, D=D, q_rows=qr, k_rows=kr, scale=D ** -0.5,
-                  q_scale=padded(gpu, qs, qr, "f32"), k_scale=padded(gpu, ks, kr, "f32"))
+                  q_scale=padded(gpu, qs, qr, "f32"), k_scale=padded(gpu, ks, kr, "f32"), **kernel)
     gpu.wait()
     got = O.numpy().astype(np.float64)
     ref = oa.ref_attention(qi * qs[..., None].astype(np.float64), ki * ks[..., None].astype(np.float64),
@@ -650,7 +664,8 @@ def test_key_count_beyond_32bit_offsets_refused(gpu):
 
 
 @pytest.mark.parametrize("path", ["int8", "bf16", "f16"])
-def test_scores_rising_far_above_the_first_block(gpu, path):
+@KERNELS
+def test_scores_rising_far_above_the_first_block(gpu, kernel, path):
     """Key scores that rise by ~100 log2 units from the first keys to the last (a ramp on one channel shared by
     every query), so that each row's reference maximum is passed by more than the accepted growth several times
     (2^30 per block with bf16 P, 2^15 with f16 P): the recomputed blocks and the rescaled O and l against float64
@@ -667,18 +682,18 @@ def test_scores_rising_far_above_the_first_block(gpu, path):
         ki, ks = q8(k)
         vb = to_bf16(v)
         got = run_attention(gpu, qi, ki, vb, dtype="bf16", Lq=Lq, L=L, H=H, KVH=H, D=D, scale=D ** -0.5, qs=qs,
-                            ks=ks, out_dt="f32")
+                            ks=ks, out_dt="f32", **kernel)
         ref = oa.ref_attention(qi * qs[..., None].astype(np.float64), ki * ks[..., None].astype(np.float64),
                                from_bf16(vb), D ** -0.5)
     elif path == "bf16":
         qb, kb, vb = to_bf16(q), to_bf16(k), to_bf16(v)
         got = run_attention(gpu, qb, kb, vb, dtype="bf16", Lq=Lq, L=L, H=H, KVH=H, D=D, scale=D ** -0.5,
-                            out_dt="f32")
+                            out_dt="f32", **kernel)
         ref = oa.ref_attention(from_bf16(qb), from_bf16(kb), from_bf16(vb), D ** -0.5)
     else:
         qh, kh, vh = q.astype(np.float16), k.astype(np.float16), v.astype(np.float16)
         got = run_attention(gpu, qh, kh, vh, dtype="f16", Lq=Lq, L=L, H=H, KVH=H, D=D, scale=D ** -0.5,
-                            out_dt="f32")
+                            out_dt="f32", **kernel)
         ref = oa.ref_attention(qh, kh, vh, D ** -0.5)
     got = got[:Lq]
     err = np.abs(got - ref)

@@ -1,5 +1,6 @@
-"""Short attention calls, which run on 32-row tiles whose waves split the keys (csrc/attention_small.hip), against
-float64 attention and against the 256-row tiles, whole (SPLIT=0) and with a split last round (GROUPS=1), on the same inputs: every head dim, score type and
+"""Short attention calls: the 32-row tiles whose waves split the keys (csrc/attention_small.hip; SMALL names them) and
+what the size chooses, against float64 attention and against the 256-row tiles, whole (SPLIT=0) and with a split last
+round (GROUPS=1), on the same inputs: every head dim, score type and
 output type, causal masks with offsets, grouped heads, batched sequences, ragged query and key counts around the
 32-key blocks and the four waves, rows reserved past the valid ones holding NaN, and rows that see no key. The
 max-abs tolerances are the attention tests' own, 5e-3 with half values and 2e-2 with bf16 (the rounding of P and of the
@@ -10,6 +11,7 @@ import numpy as np
 import pytest
 
 from h3metal_amd import ops
+from h3metal_amd.gpu import GpuError
 from oracle import attention as oa
 from oracle.bf16 import from_bf16, to_bf16
 
@@ -22,7 +24,10 @@ CASES = [  # path, D, H, KVH, Lq, L, causal, offset, sequences, output
     ("f16", 96, 2, 2, 65, 97, False, 0, 1, "bf16"), ("bf16", 96, 3, 1, 64, 64, True, 0, 1, "f16"),
     ("int8", 96, 2, 2, 40, 300, False, 0, 1, "f32"), ("f16", 64, 6, 6, 40, 40, False, 0, 3, "f16"),
     ("bf16", 64, 4, 4, 257, 31, False, 0, 2, "bf16"), ("int8", 64, 4, 2, 128, 128, True, 0, 1, "f16"),
-    ("f16", 96, 16, 16, 1500, 1500, False, 0, 1, "f16"),  # two query tiles per workgroup
+    ("f16", 64, 128, 128, 256, 256, False, 0, 32, "f16"), ("bf16", 64, 8, 4, 100, 200, False, 0, 2, "f32"),
+    ("int8", 64, 6, 6, 33, 129, False, 0, 3, "bf16"), ("f16", 64, 3, 3, 97, 130, True, 30, 1, "f32"),
+    ("f16", 96, 16, 16, 1500, 1500, False, 0, 1, "f16"), ("int8", 96, 3, 3, 129, 200, True, 71, 1, "bf16"),
+    ("bf16", 96, 4, 2, 65, 300, False, 0, 2, "bf16"),
 ]
 
 
@@ -65,7 +70,8 @@ def test_short_calls(gpu, path, D, H, KVH, Lq, L, causal, off, seqs, out):
     with np.errstate(invalid="ignore"):
         want = oa.ref_attention(qv, kv, val(vb), D ** -0.5, causal=causal, off=off)
     want = np.nan_to_num(want.reshape(Lq, H, D))  # a row that sees no key is zero
-    for variant in ({}, {"SPLIT": 0}, {"GROUPS": 1}):
+    outs = []
+    for variant in ({}, {"SPLIT": 0}, {"GROUPS": 1}, {"SMALL": 1}, *([{"SMALL": 2}] if D == 96 else [])):
         O = gpu.empty((seqs * seq_rows, sh * D), out)
         ops.attention(gpu, Q, K, V, O, Lq=Lq, L=L, H=H, KVH=KVH, D=D, q_rows=qr, k_rows=kr, scale=D ** -0.5,
                       causal=causal, causal_off=off, seq_heads=sh, seq_rows=seq_rows, **extra, **variant)
@@ -76,7 +82,21 @@ def test_short_calls(gpu, path, D, H, KVH, Lq, L, causal, off, seqs, out):
         got = o[:, :Lq].transpose(1, 0, 2, 3).reshape(Lq, H, D)
         err = np.abs(got - want)
         assert np.isfinite(got).all(), variant
+        outs.append(got)
         assert err.max() < (5e-3 if path == "f16" and out != "bf16" else 2e-2) and err.mean() < 2 ** -9, (variant, err.max())
+    if D == 96:  # two query tiles per workgroup: each row's keys, waves and merge are those of one
+        assert np.array_equal(outs[4], outs[3])
+
+
+def test_small_macro_refusals(gpu):
+    """SMALL is 1, or 2 at head dim 96, and names a kernel: not beside SPLIT=0 or GROUPS=1, nor for the scores hook where
+    that runs another one."""
+    for fn, m in (("attention", dict(HD=128, SMALL=2)), ("attention", dict(HD=96, SMALL=3)),
+                  ("attention", dict(HD=64, SMALL=-1)), ("attention", dict(HD=128, SMALL=1, SPLIT=0)),
+                  ("attention", dict(HD=128, SMALL=1, GROUPS=1)), ("attention_scores", dict(HD=64, SMALL=1)),
+                  ("attention_scores", dict(HD=128, SMALL=1, CAUSAL=1))):
+        with pytest.raises(GpuError, match="SMALL"):
+            gpu.kernel("attention", fn, **m)
 
 
 @pytest.mark.parametrize("path,D,H,Lq,L", [("int8", 128, 4, 32, 20000), ("bf16", 128, 1, 200, 20000),

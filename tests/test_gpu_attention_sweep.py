@@ -1,7 +1,7 @@
 """A seeded sweep of attention shapes through ops.attention against float64 attention of the same (dequantised
 or rounded) inputs (the reference's tests/test_attention.py:9-21 convention), at the north-star tolerance:
-random head counts (up to 600 one-tile heads, so that the tail split, the XCD order and the reversed key order
-of later rounds all occur), GQA ratios, ragged query and key counts, int8 (rotation-free per-row codes with
+on the wave-pipelined kernel (GROUPS=1) and on what the call's size chooses, random head counts (up to 600 one-tile
+heads, so that the tail split, the XCD order and the reversed key order of later rounds all occur), GQA ratios, ragged query and key counts, int8 (rotation-free per-row codes with
 outlier channels) and bf16 / f16 inputs, and all three output types. Every case prints its parameters before
 it runs."""
 
@@ -72,13 +72,14 @@ def test_random_shape_against_float64(gpu, seed):
         qh, kh, vh = xq.astype(np.float16), xk.astype(np.float16), xv.astype(np.float16)
         Q, K, V = padded(gpu, qh, q_rows, "f16"), padded(gpu, kh, k_rows, "f16"), padded(gpu, vh, k_rows, "f16")
         qr, kr, vr = qh, kh, vh
-    O = gpu.empty((q_rows, H * D), out_dt)
-    ops.attention(gpu, Q, K, V, O, Lq=Lq, L=L, H=H, KVH=KVH, D=D, q_rows=q_rows, k_rows=k_rows, scale=D ** -0.5,
-                  **extra)
-    gpu.wait()
-    o = O.numpy()[:Lq]
-    got = from_bf16(o) if out_dt == "bf16" else o.astype(np.float64)
     ref = oa.ref_attention(qr, kr, vr, D ** -0.5)
-    err = np.abs(got.astype(np.float64) - ref)
-    assert np.isfinite(got).all()
-    assert err.max() < NS_MAX and err.mean() < NS_MEAN, (err.max(), err.mean())
+    for groups in (0, 1):
+        O = gpu.empty((q_rows, H * D), out_dt)
+        ops.attention(gpu, Q, K, V, O, Lq=Lq, L=L, H=H, KVH=KVH, D=D, q_rows=q_rows, k_rows=k_rows, scale=D ** -0.5,
+                      GROUPS=groups, **extra)
+        gpu.wait()
+        o = O.numpy()[:Lq]
+        got = from_bf16(o) if out_dt == "bf16" else o.astype(np.float64)
+        err = np.abs(got.astype(np.float64) - ref)
+        assert np.isfinite(got).all(), groups
+        assert err.max() < NS_MAX and err.mean() < NS_MEAN, (groups, err.max(), err.mean())
