@@ -354,6 +354,8 @@ __global__ __launch_bounds__(256) void widen_i8_f16(const signed char *__restric
   *(f16x8 *)(out + n * K + k) = h;
 }
 
+enum { TILE_KSPLIT = 1, TILE_128 = TILE_KSPLIT + 4, TILE_256 };  // values of the macro TILE, 0 the plan's choice
+
 // How a product runs: which tiles, and for the 256 x 256 ones how many rows its main launch takes (the trailing rows
 // then run as 128 x 128 tiles).
 struct Plan {
@@ -366,12 +368,17 @@ struct Plan {
 // that is linear in the bytes of a row of A's K: us = fixed + per_kb * K bytes / 1024, fitted to a sweep of 3 formats
 // x 11 row counts (16 to 3300) x 5 (N, K) pairs (N 1024 to 12288, K 1024 to 10240) on an MI355X; the plan's time was
 // within 1% of the best configuration's on average over the sweep, 1.31x of it at worst, and never above that of
-// the 256 x 256 tiles with their tail launch (which it beat 2.8x on average). 256 x 256 tiles: when the last round of tiles would leave more than
-// half the CUs idle, its rows may go to a second launch of 128 x 128 tiles (0.45 of a big tile's time each).
+// the 256 x 256 tiles with their tail launch (which it beat 2.8x on average). 256 x 256 tiles: when the last round of
+// tiles would leave more than half the CUs idle, its rows may go to a second launch of 128 x 128 tiles (0.45 of a big
+// tile's time each).
 // h8 outside gemm_ksplit.hip also widens its weights first (about 14 us for 4096 x 4096).
-Plan make_plan(const GemmParams &p, int wfmt, int es, bool can_ksplit) {
+// `tile` names one (TILE_*): that, its tail launch included, whatever its time.
+Plan make_plan(const GemmParams &p, int wfmt, int es, bool can_ksplit, int tile) {
   Plan pl;
   pl.main_rows = p.M;
+  if (tile >= TILE_KSPLIT && tile < TILE_128) pl.ksplit = tile - TILE_KSPLIT;
+  if (tile == TILE_128) pl.small = true;
+  if (tile && tile != TILE_256) return pl;
   const int cus = cu_count();
   if (cus <= 0) return pl;
   const double kb = (double)p.K * es / 1024, widen = wfmt == 6 ? 3 + 0.7e-6 * (double)p.N * p.K : 0;
@@ -388,6 +395,7 @@ Plan make_plan(const GemmParams &p, int wfmt, int es, bool can_ksplit) {
   }
   // the smaller tiles have to be estimated 12% faster: near the line the estimate's error decides, and the residual
   // form, whose end costs more on small tiles, lost 7% there
+  if (tile) return pl;
   double best = 0.88 * (widen + r * (9.5 + 9.5 * kb));
   const double small = widen + rounds(tiles(p.M, ST, ST)) * (4.0 + 3.7 * kb);
   if (small < best) best = small, pl.small = true;
@@ -406,7 +414,6 @@ Plan make_plan(const GemmParams &p, int wfmt, int es, bool can_ksplit) {
 template <int OT, int EPI, bool HAS_BIAS, int WFMT>
 int launch_gemm(const Pipeline &pl, const Exec &ex, const Arg *a, int nargs, const void *params,
                 uint32_t params_len, std::string *err) {
-  (void)pl;
   constexpr int AT = WFMT == 1 ? A_I8 : WFMT == 5 ? A_BF16 : A_F16;
   constexpr int SM = WFMT == 1 ? S_ROW_COL : WFMT == 6 ? S_COL : S_NONE;
   constexpr int ES = AT == A_I8 ? 1 : 2;             // bytes per A element
@@ -477,7 +484,12 @@ int launch_gemm(const Pipeline &pl, const Exec &ex, const Arg *a, int nargs, con
   const bool vec = al16(a[4].ptr) && (p.c_stride * OSZ) % 16 == 0 && p.N % VE == 0 &&
                    (SM == S_NONE || al16(a[2].ptr)) && (!HAS_BIAS || al16(a[5].ptr)) &&
                    (!EPI || (al16(a[7].ptr) && p.g_stride % 4 == 0));
-  const Plan plan = make_plan(p, WFMT, ES, WFMT != 6 || p.w_stride % 16 == 0);
+  const bool can_ksplit = WFMT != 6 || p.w_stride % 16 == 0;
+  const Plan plan = make_plan(p, WFMT, ES, can_ksplit, pl.ival[0]);
+  if (plan.ksplit >= 0 && !can_ksplit) {
+    *err = "TILE " + std::to_string(pl.ival[0]) + " needs 16-byte rows of int8 weights";
+    return -1;
+  }
   if (plan.ksplit >= 0) {
     const GemmArgs g{a[0].ptr,
                      a[1].ptr,
@@ -545,21 +557,24 @@ LaunchFn pick(int epi, int ot, bool bias) {
 
 // Macros (those of h3metal/ops.py:161-164): WFMT (1 q8, 4 f16, 5 bf16, 6 h8), EPI (0 or 1), OUT_T (half | bfloat |
 // float; float for EPI 1), HAS_BIAS. The reference's tile and layout choices TM, TN, NSG, G, SWZ, FAST_LAYOUT
-// are accepted and unused (this kernel's tiles are its own); LORA must be 0.
+// are accepted and unused (this kernel's tiles are its own); LORA must be 0. TILE (this build's, default 0: what is
+// estimated fastest) names the tiles at every size: 1 to 4 the 32 x 32, 64 x 64, 96 x 64 and (16-bit activations)
+// 96 x 128 tiles whose waves split K, 5 128 x 128, 6 256 x 256 and their tail launch.
 bool make_gemm(const std::string &fn, const Macros &m, Pipeline *pl, std::string *err) {
   if (fn != "gemm") {
     *err = "unknown function (have: gemm)";
     return false;
   }
-  int wfmt, epi, hb, lora, dummy;
+  int wfmt, epi, hb, lora, tile, dummy;
   if (!macro_int(m, "WFMT", 1, &wfmt, err) || !macro_int(m, "EPI", 0, &epi, err) ||
-      !macro_int(m, "HAS_BIAS", 0, &hb, err) || !macro_int(m, "LORA", 0, &lora, err))
+      !macro_int(m, "HAS_BIAS", 0, &hb, err) || !macro_int(m, "LORA", 0, &lora, err) ||
+      !macro_int(m, "TILE", 0, &tile, err))
     return false;
   for (const char *k : {"TM", "TN", "NSG", "G", "SWZ", "FAST_LAYOUT"})
     if (!macro_int(m, k, 0, &dummy, err)) return false;
   for (auto &kv : m) {
     static const char *known[] = {"WFMT", "EPI", "OUT_T", "HAS_BIAS", "LORA", "TM", "TN", "NSG", "G", "SWZ",
-                                  "FAST_LAYOUT"};
+                                  "FAST_LAYOUT", "TILE"};
     bool ok = false;
     for (const char *k : known) ok = ok || kv.first == k;
     if (!ok) {
@@ -579,6 +594,10 @@ bool make_gemm(const std::string &fn, const Macros &m, Pipeline *pl, std::string
     *err = "EPI must be 0 or 1";
     return false;
   }
+  if (tile < 0 || tile > TILE_256 || (wfmt == 1 && tile == TILE_KSPLIT + KSPLIT_96x128)) {
+    *err = "TILE must be 0 to 6, and not 4 (96 x 128) with int8 activations";
+    return false;
+  }
   const std::string t = macro_str(m, "OUT_T", epi ? "float" : "half");
   int ot = t == "bfloat" || t == "bf16" ? T_BF16 : t == "half" || t == "f16" ? T_F16 : t == "float" || t == "f32" ? T_F32 : -1;
   if (ot < 0 || (epi == 1 && ot != T_F32)) {
@@ -590,6 +609,7 @@ bool make_gemm(const std::string &fn, const Macros &m, Pipeline *pl, std::string
                : wfmt == 5 ? pick<5>(epi, ot, hb != 0)
                            : pick<6>(epi, ot, hb != 0);
   pl->threads = NWG * 64;
+  pl->ival[0] = tile;
   return true;
 }
 

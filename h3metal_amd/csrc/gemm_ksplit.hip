@@ -98,8 +98,7 @@ __global__ __launch_bounds__(C::NWK * 64) void gemm_ksplit_kernel(GemmArgs g, Ge
   const __amdgpu_buffer_rsrc_t rw =
       __builtin_amdgcn_make_buffer_rsrc((void *)(g.w + (size_t)n0 * wstr), (short)0, recw, 0x00020000);
   const int nk = (p.K * ES + KS - 1) / KS;          // K slices (the last may be half of one)
-  const int steps = (nk + NWK - 1) / NWK;
-           // of each wave (slices past the last read as zero)
+  const int steps = (nk + NWK - 1) / NWK;           // of each wave (slices past the last read as zero)
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem + w * (NST * C::SLOT);
   const char *own = smem + w * (NST * C::SLOT);
 

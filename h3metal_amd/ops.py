@@ -67,8 +67,8 @@ def attention_scores(gpu: Gpu, q: Tensor, k: Tensor, v: Tensor, scores: Tensor, 
     of its MFMAs, scores[h][i][j] = q_i . k_j (int32 for int8 inputs, f32 otherwise) for keys j < L. At D = 128
     without a causal mask the kernel that runs is ops.attention's own (the small tiles of short calls or the
     wave-pipelined kernel: same tiles, staging, split and P V), which then also writes `out` ([Lq][H * D] rows, as
-    ops.attention with seq_heads = H). GROUPS=1 selects the wave-pipelined kernel at every size. Other head dims run
-    the two-group kernel, which writes the scores only."""
+    ops.attention with seq_heads = H). GROUPS=1 selects the wave-pipelined kernel at every size, SMALL=1 the small
+    tiles. Other head dims run the two-group kernel, which writes the scores only."""
     q8 = q_scale is not None
     vt = v.dtype if v.dtype in ("f16", "bf16") else "bf16"
     if out is None:
@@ -147,7 +147,7 @@ class QWeight:
 def gemm(gpu: Gpu, a: Tensor, wt: QWeight, out: Tensor, M: int, *, sa: Tensor | None = None, epi: int = 0,
          rtype: Tensor | None = None, gate: Tensor | None = None, g_stride: int = 0, c_stride: int | None = None,
          a_stride: int | None = None, tile=(64, 128, 4), swz: int = 1, ksplit: int = 1, no_alloc: bool = False,
-         _low=None):
+         _low=None, **variant):
     """out = A x W^T (epi 0), or out += gate[rtype] * (A x W^T) (epi 1, out float), plus bias[n]:
       q8:  A int8 [M][K] with row scales sa, W int8 codes, v = sa[m] * sw[n] * (a_m . w_n)
       h8:  A half, W int8 codes, v = sw[n] * (a_m . w_n)
@@ -155,7 +155,8 @@ def gemm(gpu: Gpu, a: Tensor, wt: QWeight, out: Tensor, M: int, *, sa: Tensor | 
 
     ksplit: accumulate over that many consecutive slices of K in separate dispatches (epi 1 only), as the
     reference does. tile / swz are the Metal kernel's tile choices: checked as the reference checks them (the
-    tile width must divide N) and otherwise unused (the gfx950 kernel uses 256 x 256 tiles and covers any N).
+    tile width must divide N) and otherwise unused (the gfx950 kernels have tiles of their own, chosen by the size, and
+    cover any N). variant: TILE names those tiles (csrc/gemm.hip: make_gemm).
     no_alloc: dispatch through the allocation-free entry point (h3_dispatch_static); the h8 format's widened
     weights then live in its fixed scratch array."""
     if wt.fmt not in GEMM_ACT:
@@ -173,7 +174,7 @@ def gemm(gpu: Gpu, a: Tensor, wt: QWeight, out: Tensor, M: int, *, sa: Tensor | 
                            bias=wt.bias if i == 0 else None)
             gemm(gpu, a.view((a.shape[0], kp), offset_elems=i * kp), part, out, M, sa=sa, epi=1, rtype=rtype,
                  gate=gate, g_stride=g_stride, c_stride=c_stride, a_stride=a_stride or wt.K, tile=tile, swz=swz,
-                 no_alloc=no_alloc)
+                 no_alloc=no_alloc, **variant)
         return
     tm, tn, nsg = tile
     if wt.N % tn:
@@ -182,7 +183,7 @@ def gemm(gpu: Gpu, a: Tensor, wt: QWeight, out: Tensor, M: int, *, sa: Tensor | 
         raise ValueError("gemm: int8 activations need their row scales sa")
     out_t = OUT_DT[out.dtype] if epi == 0 else "float"
     k = gpu.kernel("gemm", "gemm", WFMT=FMT_ID[wt.fmt], EPI=epi, OUT_T=out_t, TM=tm, TN=tn, NSG=nsg, G=wt.G,
-                   HAS_BIAS=int(wt.bias is not None), SWZ=swz)
+                   HAS_BIAS=int(wt.bias is not None), SWZ=swz, **variant)
     if wt.fmt == "h8":
         gpu.reserve_workspace(wt.N * wt.K * 2)  # the widened weights; grows (and waits) only the first time
     m_pad = (M + tm - 1) // tm * tm

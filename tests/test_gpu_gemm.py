@@ -13,6 +13,9 @@ from oracle.bf16 import from_bf16, to_bf16
 
 pytestmark = pytest.mark.gpu
 
+# the plan's own choice (at these sizes one of the K-split tiles), 128 x 128 and 256 x 256 tiles
+PLANS = pytest.mark.parametrize("TILE", [0, 5, 6], ids=["plan", "128x128", "256x256"])
+
 
 def make(rng, M, N, K, m_pad=None, bias=False):
     m_pad = m_pad or M
@@ -24,7 +27,7 @@ def make(rng, M, N, K, m_pad=None, bias=False):
     return a, sa, q, sw, b
 
 
-def run(gpu, a, sa, q, sw, b, M, out_dtype="f32", tile=(64, 128, 4), no_alloc=False):
+def run(gpu, a, sa, q, sw, b, M, out_dtype="f32", tile=(64, 128, 4), no_alloc=False, **variant):
     N, K = q.shape
     print(f"[gemm] M={M} N={N} K={K} out={out_dtype} bias={b is not None}", flush=True)
     wt = ops.QWeight("q8", gpu.upload(q), gpu.upload(sw), N, K, bias=gpu.upload(b) if b is not None else None)
@@ -32,7 +35,7 @@ def run(gpu, a, sa, q, sw, b, M, out_dtype="f32", tile=(64, 128, 4), no_alloc=Fa
     A = gpu.upload(np.pad(a, ((0, max(0, m_pad - a.shape[0])), (0, 0))))
     SA = gpu.upload(np.pad(sa, (0, max(0, m_pad - sa.shape[0]))))
     out = gpu.empty((m_pad, N), out_dtype)
-    ops.gemm(gpu, A, wt, out, M, sa=SA, tile=tile, no_alloc=no_alloc)
+    ops.gemm(gpu, A, wt, out, M, sa=SA, tile=tile, no_alloc=no_alloc, **variant)
     gpu.wait()
     return out.numpy()[:M]
 
@@ -40,20 +43,22 @@ def run(gpu, a, sa, q, sw, b, M, out_dtype="f32", tile=(64, 128, 4), no_alloc=Fa
 @pytest.mark.parametrize("M,N,K,bias", [(200, 256, 512, False), (300, 640, 384, True), (64, 1024, 128, True),
                                         (1, 256, 256, False), (513, 512, 1280, False),
                                         (70, 256, 64, True), (130, 512, 192, False)])
-def test_f32_outputs_bit_exact(gpu, M, N, K, bias):
+@PLANS
+def test_f32_outputs_bit_exact(gpu, TILE, M, N, K, bias):
     rng = np.random.default_rng(M + N + K)
     a, sa, q, sw, b = make(rng, M, N, K, bias=bias)
-    got = run(gpu, a, sa, q, sw, b, M)
+    got = run(gpu, a, sa, q, sw, b, M, TILE=TILE)
     want = og.epilogue(og.int_product(a[:M], q), sa[:M], sw, b)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
 @pytest.mark.parametrize("out_dtype", ["f16", "bf16"])
-def test_16bit_outputs_are_the_rounded_oracle(gpu, out_dtype):
+@PLANS
+def test_16bit_outputs_are_the_rounded_oracle(gpu, TILE, out_dtype):
     rng = np.random.default_rng(41)
     M, N, K = 250, 512, 768
     a, sa, q, sw, b = make(rng, M, N, K, bias=True)
-    got = run(gpu, a, sa, q, sw, b, M, out_dtype=out_dtype)
+    got = run(gpu, a, sa, q, sw, b, M, out_dtype=out_dtype, TILE=TILE)
     v = og.epilogue(og.int_product(a, q), sa, sw, b)
     if out_dtype == "bf16":
         assert np.array_equal(got, to_bf16(v))
@@ -62,13 +67,14 @@ def test_16bit_outputs_are_the_rounded_oracle(gpu, out_dtype):
 
 
 @pytest.mark.parametrize("N,out_dtype", [(200, "f16"), (198, "bf16"), (198, "f32"), (260, "f32")])
-def test_ragged_columns_element_path(gpu, N, out_dtype):
+@PLANS
+def test_ragged_columns_element_path(gpu, TILE, N, out_dtype):
     """Column counts that are not a multiple of the 16-byte vector (and partial column tiles): the kernel's
     per-element output path, bit-exact."""
     rng = np.random.default_rng(N)
     M, K = 70, 192
     a, sa, q, sw, b = make(rng, M, N, K, bias=True)
-    got = run(gpu, a, sa, q, sw, b, M, out_dtype=out_dtype, tile=(64, 2, 4))
+    got = run(gpu, a, sa, q, sw, b, M, out_dtype=out_dtype, tile=(64, 2, 4), TILE=TILE)
     v = og.epilogue(og.int_product(a[:M], q), sa[:M], sw, b)
     if out_dtype == "f32":
         assert np.array_equal(got.view(np.uint32), v.view(np.uint32))
@@ -78,7 +84,8 @@ def test_ragged_columns_element_path(gpu, N, out_dtype):
         assert np.array_equal(got.view(np.uint16), v.astype(np.float16).view(np.uint16))
 
 
-def test_residual_ragged_columns_and_strided_output(gpu):
+@PLANS
+def test_residual_ragged_columns_and_strided_output(gpu, TILE):
     """epi 1 with N = 198 into a residual buffer with a wider row stride (c_stride 203): element path; the
     columns past N are left alone."""
     rng = np.random.default_rng(5)
@@ -90,7 +97,7 @@ def test_residual_ragged_columns_and_strided_output(gpu):
     wt = ops.QWeight("q8", gpu.upload(q), gpu.upload(sw), N, K, bias=gpu.upload(b))
     X = gpu.upload(x0)
     ops.gemm(gpu, gpu.upload(a), wt, X, M, sa=gpu.upload(sa), epi=1, rtype=gpu.upload(types),
-             gate=gpu.upload(gates), c_stride=CS, tile=(64, 2, 4))
+             gate=gpu.upload(gates), c_stride=CS, tile=(64, 2, 4), TILE=TILE)
     gpu.wait()
     v = og.epilogue(og.int_product(a, q), sa, sw, b)
     want = x0.copy()
@@ -98,7 +105,8 @@ def test_residual_ragged_columns_and_strided_output(gpu):
     assert np.array_equal(X.numpy().view(np.uint32), want.view(np.uint32))
 
 
-def test_residual_epilogue_bit_exact_and_k_split(gpu):
+@PLANS
+def test_residual_epilogue_bit_exact_and_k_split(gpu, TILE):
     """epi 1: X += gate[rtype] * v, exact in one dispatch; with K split over 4 dispatches (the reference's ksplit),
     each slice's product is added in turn, which the oracle reproduces slice by slice."""
     rng = np.random.default_rng(42)
@@ -111,7 +119,7 @@ def test_residual_epilogue_bit_exact_and_k_split(gpu):
     A, SA, RT, GT = gpu.upload(a), gpu.upload(sa), gpu.upload(types), gpu.upload(gates)
     for ksplit in (1, 4):
         X = gpu.upload(x0)
-        ops.gemm(gpu, A, wt, X, M, sa=SA, epi=1, rtype=RT, gate=GT, ksplit=ksplit, tile=(64, 256, 8))
+        ops.gemm(gpu, A, wt, X, M, sa=SA, epi=1, rtype=RT, gate=GT, ksplit=ksplit, tile=(64, 256, 8), TILE=TILE)
         gpu.wait()
         want = x0
         kp = K // ksplit
@@ -125,7 +133,8 @@ def test_residual_epilogue_bit_exact_and_k_split(gpu):
 @pytest.mark.parametrize("case", [dict(), dict(out_dtype="bf16"), dict(epi=1, K=2048, ksplit=4, tile=(64, 256, 8)),
                                   dict(N=1024, tile=(32, 512, 8)), dict(epi=1, N=1024, K=2048, ksplit=4,
                                                                           tile=(32, 512, 8))])
-def test_reference_check_cases(gpu, case):
+@PLANS
+def test_reference_check_cases(gpu, TILE, case):
     """check() of tests/test_gemm.py:20-84 for the q8 format: max relative error against float64 below 2e-3
     (1e-2 for bf16 outputs)."""
     c = dict(M=200, N=256, K=512, epi=0, out_dtype="f16", tile=(64, 128, 4), ksplit=1)
@@ -141,7 +150,7 @@ def test_reference_check_cases(gpu, case):
     A, SA = gpu.upload(a), gpu.upload(sa)
     if c["epi"] == 0:
         out = gpu.empty((m_pad, c["N"]), c["out_dtype"])
-        ops.gemm(gpu, A, wt, out, c["M"], sa=SA, tile=c["tile"])
+        ops.gemm(gpu, A, wt, out, c["M"], sa=SA, tile=c["tile"], TILE=TILE)
         gpu.wait()
         got = out.numpy()[:c["M"]]
         got = from_bf16(got).astype(np.float64) if c["out_dtype"] == "bf16" else got.astype(np.float64)
@@ -151,7 +160,7 @@ def test_reference_check_cases(gpu, case):
         types = rng.integers(0, 3, size=m_pad).astype(np.uint8)
         gates = rng.standard_normal((3, c["N"])).astype(np.float32)
         ops.gemm(gpu, A, wt, X, c["M"], sa=SA, epi=1, rtype=gpu.upload(types), gate=gpu.upload(gates),
-                 tile=c["tile"], ksplit=c["ksplit"])
+                 tile=c["tile"], ksplit=c["ksplit"], TILE=TILE)
         gpu.wait()
         got = X.numpy()[:c["M"]].astype(np.float64)
         ref = x0.astype(np.float64) + gates[types] * ref
@@ -178,7 +187,7 @@ def test_config4_projection_shapes_sampled(gpu):
 @pytest.mark.parametrize("mode", ["f32", "bf16", "epi1"])
 @pytest.mark.parametrize("no_alloc", [False, True])
 def test_last_round_rows_on_small_tiles(gpu, mode, no_alloc):
-    """260 tiles of 256 x 256 on 256 CUs: the last row of tiles (rows 16384..16447) runs as a second launch of
+    """260 tiles of 256 x 256 (TILE 6) on 256 CUs: the last row of tiles (rows 16384..16447) runs as a second launch of
     128 x 128 tiles on the sub-problem of those rows; every row bit for bit (f32, the residual form) or equal to
     the rounded oracle (bf16), the rows of both launches alike; through h3_dispatch and through the
     allocation-free entry point h3_dispatch_static."""
@@ -194,12 +203,12 @@ def test_last_round_rows_on_small_tiles(gpu, mode, no_alloc):
         X = gpu.upload(x0)
         print(f"[gemm] tail rows M={M} N={N} K={K} epi=1 no_alloc={no_alloc}", flush=True)
         ops.gemm(gpu, gpu.upload(a), wt, X, M, sa=gpu.upload(sa), epi=1, rtype=gpu.upload(types),
-                 gate=gpu.upload(gates), tile=(64, 256, 8), no_alloc=no_alloc)
+                 gate=gpu.upload(gates), tile=(64, 256, 8), no_alloc=no_alloc, TILE=6)
         gpu.wait()
         want = og.residual(x0, v, gates, types)
         assert np.array_equal(X.numpy().view(np.uint32), want.view(np.uint32))
         return
-    got = run(gpu, a, sa, q, sw, b, M, out_dtype=mode, no_alloc=no_alloc)
+    got = run(gpu, a, sa, q, sw, b, M, out_dtype=mode, no_alloc=no_alloc, TILE=6)
     if mode == "f32":
         assert np.array_equal(got.view(np.uint32), v.view(np.uint32))
     else:
@@ -315,7 +324,8 @@ def float_case(gpu, fmt, rng, M, N, K, bias):
 @pytest.mark.parametrize("fmt", ["h8", "f16", "bf16"])
 @pytest.mark.parametrize("M,N,K,out_dtype,bias", [(200, 256, 512, "f16", False), (300, 640, 384, "f32", True),
                                                   (70, 198, 96, "bf16", True), (513, 512, 1280, "f32", False)])
-def test_float_formats_reference_tolerance(gpu, fmt, M, N, K, out_dtype, bias):
+@PLANS
+def test_float_formats_reference_tolerance(gpu, TILE, fmt, M, N, K, out_dtype, bias):
     """h8 / f16 / bf16 products (WFMT 6 / 4 / 5) within the reference's check() tolerance (tests/test_gemm.py:
     20-84): max error below 2e-3 of the largest output, 1e-2 for bfloat outputs; ragged N and a K of three
     32-element steps included."""
@@ -323,7 +333,7 @@ def test_float_formats_reference_tolerance(gpu, fmt, M, N, K, out_dtype, bias):
     print(f"[gemm {fmt}] M={M} N={N} K={K} out={out_dtype} bias={bias}", flush=True)
     A, wt, v = float_case(gpu, fmt, rng, M, N, K, bias)
     out = gpu.empty((M, N), out_dtype)
-    ops.gemm(gpu, A, wt, out, M, tile=(1, 2, 4))
+    ops.gemm(gpu, A, wt, out, M, tile=(1, 2, 4), TILE=TILE)
     gpu.wait()
     got = out.numpy()
     got = from_bf16(got).astype(np.float64) if out_dtype == "bf16" else got.astype(np.float64)
@@ -332,7 +342,8 @@ def test_float_formats_reference_tolerance(gpu, fmt, M, N, K, out_dtype, bias):
 
 
 @pytest.mark.parametrize("fmt", ["h8", "f16", "bf16"])
-def test_float_formats_residual_and_k_split(gpu, fmt):
+@PLANS
+def test_float_formats_residual_and_k_split(gpu, TILE, fmt):
     """epi 1 with row types and gates; h8 also with K split over dispatches (the reference allows it for h8)."""
     rng = np.random.default_rng(7)
     M, N, K = 256, 512, 1024
@@ -344,13 +355,14 @@ def test_float_formats_residual_and_k_split(gpu, fmt):
     for ksplit in ((1, 4) if fmt == "h8" else (1,)):
         X = gpu.upload(x0)
         ops.gemm(gpu, A, wt, X, M, epi=1, rtype=gpu.upload(types), gate=gpu.upload(gates), ksplit=ksplit,
-                 tile=(64, 256, 8))
+                 tile=(64, 256, 8), TILE=TILE)
         gpu.wait()
         err = np.abs(X.numpy().astype(np.float64) - want).max() / np.abs(want).max()
         assert err < 2e-3, (fmt, ksplit, err)
 
 
-def test_rotated_half_output_into_h8_projection(gpu):
+@PLANS
+def test_rotated_half_output_into_h8_projection(gpu, TILE):
     """The text encoder's chain (h3metal/te.py:195-196): rot_q8 with out_hr (rotated rows in half precision)
     feeding an h8 projection; against float64 of the rotated rows."""
     from oracle import rot_q8 as orq
@@ -364,7 +376,7 @@ def test_rotated_half_output_into_h8_projection(gpu):
     sw = rng.uniform(0.001, 0.01, size=N).astype(np.float32)
     wt = ops.QWeight("h8", gpu.upload(q), gpu.upload(sw), N, D)
     out = gpu.empty((M, N), "f32")
-    ops.gemm(gpu, hr, wt, out, M, tile=(1, 2, 4))
+    ops.gemm(gpu, hr, wt, out, M, tile=(1, 2, 4), TILE=TILE)
     gpu.wait()
     _, _, r = orq.rot_q8(from_bf16(xb), D)
     want = og.float_product(r.astype(np.float16).astype(np.float32), q) * sw[None, :].astype(np.float64)
@@ -385,15 +397,25 @@ def test_float_format_refusals(gpu):
         ops.gemm(gpu, A, ops.QWeight("f16", wt.w, None, 256, 200, ws=256), out, 64, a_stride=256, tile=(1, 2, 4))
 
 
-@pytest.mark.parametrize("fmt", ["q8", "h8", "bf16"])
-@pytest.mark.parametrize("M,N,K", [(1, 36, 64), (33, 1000, 1088), (130, 4096, 1088), (97, 8192, 192),
-                                   (289, 4096, 1088), (385, 4100, 2112)])
-def test_few_tiles_bit_exact(gpu, fmt, M, N, K):
-    """Products of few output tiles (the waves of a workgroup split K): each small tile (32 x 32, 64 x 64, 96 x 64,
-    and for h8 at 385 rows 96 x 128) with ragged rows and columns, fewer K slices than waves and a last half slice.
-    The operands are small integers, so every format's sums are whole numbers below 2^24, exact in float32 in any
-    order, and both epilogues are compared bit for bit."""
-    rng = np.random.default_rng(M + N + K)
+def test_tile_macro_refusals(gpu):
+    """TILE names one of the six tile choices, of which int8 activations have no 96 x 128; the K-split tiles take int8
+    weights of half activations in 16-byte rows only (checked at the launch)."""
+    for wfmt, tile in ((1, -1), (1, 7), (6, 7), (1, 4)):
+        with pytest.raises(GpuError, match="TILE"):
+            gpu.kernel("gemm", "gemm", WFMT=wfmt, TILE=tile)
+    w = gpu.upload(np.zeros((64, 136), np.int8))
+    wt = ops.QWeight("h8", w, gpu.upload(np.ones(64, np.float32)), 64, 128, ws=136)
+    a, out = gpu.upload(np.zeros((64, 128), np.float16)), gpu.empty((64, 64), "f16")
+    for tile in (1, 2, 3, 4):
+        with pytest.raises(GpuError, match="16-byte rows"):
+            ops.gemm(gpu, a, wt, out, 64, tile=(1, 2, 4), TILE=tile)
+    ops.gemm(gpu, a, wt, out, 64, tile=(1, 2, 4))
+    gpu.wait()
+
+
+def whole_numbers(gpu, fmt, rng, M, N, K):
+    """Operands that are small integers, so that every format's sums are whole numbers below 2^24, exact in float32 in any
+    order, and a bias: the device operands (A, its scales, the weight) and the product with scales and bias in float32."""
     a = rng.integers(-8, 9, size=(M, K), dtype=np.int8)
     q = rng.integers(-127, 128, size=(N, K), dtype=np.int8)
     assert K * 8 * 127 < 2 ** 24
@@ -404,18 +426,48 @@ def test_few_tiles_bit_exact(gpu, fmt, M, N, K):
         A, W, v = gpu.upload(a), gpu.upload(q), og.epilogue(acc, sa, sw, b)
     elif fmt == "h8":
         A, W, v = gpu.upload(a.astype(np.float16)), gpu.upload(q), acc.astype(np.float32) * sw + b
+    elif fmt == "f16":
+        A, W = (gpu.upload(t.astype(np.float16)) for t in (a, q))
+        v = acc.astype(np.float32) + b
     else:
         A, W = (gpu.upload(to_bf16(t.astype(np.float32)), "bf16") for t in (a, q))
         v = acc.astype(np.float32) + b
-    wt = ops.QWeight(fmt, W, gpu.upload(sw) if fmt != "bf16" else None, N, K, bias=gpu.upload(b))
+    wt = ops.QWeight(fmt, W, gpu.upload(sw) if fmt in ("q8", "h8") else None, N, K, bias=gpu.upload(b))
+    return A, gpu.upload(sa) if fmt == "q8" else None, wt, v
+
+
+def check_whole_numbers(gpu, rng, A, SA, wt, v, tile):
+    """Both epilogues on tile choice `tile`, bit for bit."""
+    M, N = v.shape
     out, x0 = gpu.empty((M, N), "f32"), rng.standard_normal((M, N)).astype(np.float32)
     types = rng.integers(0, 3, size=M).astype(np.uint8)
     gates = rng.standard_normal((3, N)).astype(np.float32)
     X = gpu.upload(x0)
-    SA = gpu.upload(sa) if fmt == "q8" else None
-    print(f"[gemm few tiles] {fmt} M={M} N={N} K={K}", flush=True)
-    ops.gemm(gpu, A, wt, out, M, sa=SA, tile=(1, 2, 4))
-    ops.gemm(gpu, A, wt, X, M, sa=SA, epi=1, rtype=gpu.upload(types), gate=gpu.upload(gates), tile=(1, 2, 4))
+    print(f"[gemm whole numbers] {wt.fmt} M={M} N={N} K={wt.K} TILE={tile}", flush=True)
+    ops.gemm(gpu, A, wt, out, M, sa=SA, tile=(1, 2, 4), TILE=tile)
+    ops.gemm(gpu, A, wt, X, M, sa=SA, epi=1, rtype=gpu.upload(types), gate=gpu.upload(gates), tile=(1, 2, 4), TILE=tile)
     gpu.wait()
-    assert np.array_equal(out.numpy().view(np.uint32), v.view(np.uint32))
-    assert np.array_equal(X.numpy().view(np.uint32), (x0 + gates[types] * v).view(np.uint32))
+    assert np.array_equal(out.numpy().view(np.uint32), v.view(np.uint32)), tile
+    assert np.array_equal(X.numpy().view(np.uint32), (x0 + gates[types] * v).view(np.uint32)), tile
+
+
+@pytest.mark.parametrize("fmt", ["q8", "h8", "f16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1, 36, 64), (33, 1000, 1088), (130, 4096, 1088), (97, 8192, 192),
+                                   (289, 4096, 1088), (385, 4100, 2112)])
+def test_few_tiles_bit_exact(gpu, fmt, M, N, K):
+    """Products of few output tiles, on each tile choice: the tiles whose waves split K (32 x 32, 64 x 64, 96 x 64, and
+    with 16-bit activations 96 x 128, for f16 and bf16 with a single slot of the ring), 128 x 128 and 256 x 256 tiles (h8:
+    with widened weights); ragged rows and columns, fewer K slices than waves and a last half slice."""
+    rng = np.random.default_rng(M + N + K)
+    case = whole_numbers(gpu, fmt, rng, M, N, K)
+    for tile in range(7):
+        if (fmt, tile) != ("q8", 4):
+            check_whole_numbers(gpu, rng, *case, tile)
+
+
+@pytest.mark.parametrize("fmt", ["h8", "f16", "bf16"])
+def test_last_round_rows_of_float_formats(gpu, fmt):
+    """260 tiles of 256 x 256 on 256 CUs, the last row of tiles in a second launch of 128 x 128 tiles, with 16-bit
+    operands."""
+    rng = np.random.default_rng(48)
+    check_whole_numbers(gpu, rng, *whole_numbers(gpu, fmt, rng, 16448, 1024, 128), 6)

@@ -28,13 +28,13 @@ def _inputs(gpu, H, S, seed):
     return T, qi, ki
 
 
-def _attention(gpu, T, H, S, no_alloc, scores=None):
+def _attention(gpu, T, H, S, no_alloc, scores=None, **kernel):
     O = gpu.empty((S, H * D), "bf16")
     if scores is None:
-        k = gpu.kernel("attention", "attention", HD=D, QK8=1, IN_T="bfloat", O_T="bfloat")
+        k = gpu.kernel("attention", "attention", HD=D, QK8=1, IN_T="bfloat", O_T="bfloat", **kernel)
         bufs = [T["q"], T["k"], T["v"], O, None, T["qs"], T["ks"]]
     else:
-        k = gpu.kernel("attention", "attention_scores", HD=D, QK8=1, IN_T="bfloat", O_T="bfloat")
+        k = gpu.kernel("attention", "attention_scores", HD=D, QK8=1, IN_T="bfloat", O_T="bfloat", **kernel)
         bufs = [T["q"], T["k"], T["v"], O, None, T["qs"], T["ks"], scores]
     params = pack("7if3i", S, S, H, H, S, S, H * D, D ** -0.5 * ops.LOG2E, 0, H, 0)
     gpu.launch(k, None, None, bufs, params, params_index=4, no_alloc=no_alloc)
@@ -43,33 +43,35 @@ def _attention(gpu, T, H, S, no_alloc, scores=None):
 
 
 @pytest.mark.parametrize("H,S", [(1, 1024), (1, 700)])  # the second call smaller than the first
-def test_static_attention_matches_dispatch(gpu, H, S):
+@pytest.mark.parametrize("kernel", [dict(GROUPS=1), dict(SMALL=1)], ids=["split", "small"])
+def test_static_attention_matches_dispatch(gpu, H, S, kernel):
     """Both entry points split the last round of tiles the same way at these shapes (the static scratch holds
-    the split), so the outputs agree bit for bit; the scores hook through the static entry point gives exact
-    int32 products."""
+    the split), and the small tiles use no scratch, so the outputs agree bit for bit; the scores hook through the static
+    entry point gives exact int32 products."""
     T, qi, ki = _inputs(gpu, H, S, S)
-    print(f"[no-alloc] attention H={H} S={S}", flush=True)
-    want = _attention(gpu, T, H, S, no_alloc=False)
-    got = _attention(gpu, T, H, S, no_alloc=True)
+    print(f"[no-alloc] attention H={H} S={S} {kernel}", flush=True)
+    want = _attention(gpu, T, H, S, no_alloc=False, **kernel)
+    got = _attention(gpu, T, H, S, no_alloc=True, **kernel)
     assert np.array_equal(got, want)
-    again = _attention(gpu, T, H, S, no_alloc=True)  # the array keeps the last call's contents: no effect
+    again = _attention(gpu, T, H, S, no_alloc=True, **kernel)  # the array keeps the last call's contents: no effect
     assert np.array_equal(again, want)
     Sc = gpu.empty((H, S, S), "i32")
-    out = _attention(gpu, T, H, S, no_alloc=True, scores=Sc)
+    out = _attention(gpu, T, H, S, no_alloc=True, scores=Sc, **kernel)
     assert np.array_equal(Sc.numpy(), oa.int_scores(qi, ki))
     assert np.array_equal(out, want)
 
 
-def test_static_h8_gemm(gpu):
-    """The h8 GEMM's widened weights live in the static scratch: a product that fits matches h3_dispatch bit for
-    bit; one that needs more than the 32 MiB is refused with the size it needs, although the context's own
+@pytest.mark.parametrize("TILE", [0, 6])
+def test_static_h8_gemm(gpu, TILE):
+    """The h8 GEMM's widened weights live in the static scratch (TILE 6: 256 x 256 tiles; the plan's tiles here, TILE 0,
+    widen in registers and ask for the same scratch): a product that fits matches h3_dispatch bit for bit; one that needs more than the 32 MiB is refused with the size it needs, although the context's own
     workspace (grown to 48 MiB) runs it through h3_dispatch."""
     rng = np.random.default_rng(3)
     M, N, K = 64, 256, 512
     a = gpu.upload(rng.standard_normal((M, K)).astype(np.float16))
     w = gpu.upload(rng.integers(-127, 128, (N, K)).astype(np.int8), "i8")
     sw = gpu.upload(rng.uniform(1e-3, 1e-2, N).astype(np.float32))
-    k = gpu.kernel("gemm", "gemm", WFMT=6, EPI=0, OUT_T="half", TM=64, TN=128, NSG=4, G=128, HAS_BIAS=0, SWZ=1)
+    k = gpu.kernel("gemm", "gemm", WFMT=6, EPI=0, OUT_T="half", TM=64, TN=128, NSG=4, G=128, HAS_BIAS=0, SWZ=1, TILE=TILE)
 
     def run(no_alloc, n, kk, wt, out):
         gpu.launch(k, None, None, [a, wt, sw, None, out, None, None, None],
