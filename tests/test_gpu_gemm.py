@@ -471,3 +471,19 @@ def test_last_round_rows_of_float_formats(gpu, fmt):
     operands."""
     rng = np.random.default_rng(48)
     check_whole_numbers(gpu, rng, *whole_numbers(gpu, fmt, rng, 16448, 1024, 128), 6)
+
+
+@pytest.mark.parametrize("M,N,K", [(40000, 32, 256), (40000, 8, 128)])
+def test_many_short_rounds_are_not_split(gpu, M, N, K):
+    """Rows by the ten thousand with few columns and a short K, where the K-split tiles take twice the time of 128 x 128
+    ones (14.5 us against 7): the plan takes the latter, bit for bit, and the K-split tiles' sums differ."""
+    rng = np.random.default_rng(N)
+    A, W = (gpu.upload(to_bf16(rng.standard_normal((r, K)).astype(np.float32)), "bf16") for r in (M, N))
+    outs = []
+    for tile in (0, 5, 1):
+        out = gpu.empty((M, N), "f32")
+        print(f"[gemm] bf16 M={M} N={N} K={K} TILE={tile}", flush=True)
+        ops.gemm(gpu, A, ops.QWeight("bf16", W, None, N, K), out, M, tile=(1, 2, 4), TILE=tile)
+        gpu.wait()
+        outs.append(out.numpy().view(np.uint32))
+    assert np.array_equal(outs[0], outs[1]) and not np.array_equal(outs[0], outs[2])
