@@ -48,8 +48,7 @@ constexpr int RB = 256;  // rotation block
 constexpr float SILU_MIN = -87.0f;  // the lowest gate of silu()
 
 // g / (1 + exp(-g)) in float, from e = exp(-|g|) <= 1 (no overflow): g / (1 + e), or g e / (1 + e) for negative g (from
-// SILU_MIN; lower gates are computed by the caller). The
-// exponent |g| log2(e) is taken with its rounding error and the constant's second part, put back to first order (they
+// SILU_MIN; below it silu_low). The exponent |g| log2(e) is taken with its rounding error and the constant's second part, put back to first order (they
 // are below 2^-15); the quotient by 1 + e, in [1, 2], from the hardware reciprocal and one step on its
 // remainder. div_fixup gives infinities and NaN what the division gives them. The gated kernel is bound by its vector
 // instructions; expf and the compiler's division took 40 of its issue slots a value, this takes 25: 16896 rows of 4096
@@ -66,6 +65,17 @@ __device__ __forceinline__ float silu(float g) {
   // the remainder num - (1 + e) q, with what the sum lost (d - 1 is exact, and so is the difference)
   const float rem = __builtin_fmaf(-(e - (d - 1.0f)), q, __builtin_fmaf(-d, q, num));
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(rem, r, q), d, num);
+}
+
+// The same for g below SILU_MIN, where 1 + exp(g) is 1: g exp(g), from 2^32 exp(g), which is a normal float where exp(g) is
+// not. Past 88.7228 the float formula's exp(-g) is infinite and its quotient zero, and NaN for -infinity.
+__device__ __forceinline__ float silu_low(float g) {
+  constexpr float L = 1.44269504088896340736f, L2 = 1.92596303e-8f, LN2 = 0.693147180559945309417f;
+  const float t = g * L;
+  const float lo = __builtin_fmaf(g, L2, __builtin_fmaf(g, L, -t));
+  const float e0 = __builtin_amdgcn_exp2f(t + 32.0f);  // the sum is exact
+  const float e = __builtin_fmaf(e0, lo * LN2, e0);
+  return g * (g < -88.7228394f ? 0.0f : e) * 0x1p-32f;
 }
 
 template <int IN_T, bool SWIGLU, bool OUT_HR, int MAXB>
@@ -95,27 +105,29 @@ __global__ __launch_bounds__(256) void rot_q8_kernel(const char *__restrict__ in
   for (int b = 0; b < MAXB; b++) {
     const int blk = hw + 8 * b;
     if (blk >= nb) continue;  // uniform over the half wave
+    unsigned far = 0;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       float val = (float)xv[b][i];
-      if constexpr (SWIGLU) val = val * silu((float)xg[b][i]);
+      if constexpr (SWIGLU) {
+        const float g = (float)xg[b][i];
+        const unsigned bits = __builtin_bit_cast(unsigned, g);
+        far = far > bits ? far : bits;
+        val = val * silu(g);
+      }
       v[b][i] = val;
     }
     if constexpr (SWIGLU) {
-      // silu's exp(-|g|) is subnormal below -87.33, and the hardware exponential flushes it: gates below SILU_MIN, told
-      // by their sign and magnitude bits, take the library's exp and division (a normal float down to -88.7)
-      unsigned far = 0;
+      // silu's exp(-|g|) is subnormal below -87.33, and the hardware exponential flushes it: gates below SILU_MIN, told by
+      // their sign and magnitude bits, take silu_low. Rare, so its wave loads the block again (kept until here, values
+      // and gates took 16 more registers: 5-10% at short rows)
+      if (__builtin_expect(__any(far > __builtin_bit_cast(unsigned, SILU_MIN)), 0)) {
+        int at = blk * RB + l32 * 8;
+        asm volatile("" : "+v"(at));  // not the loads above
+        const IV x = *(const IV *)(row + at), gt = *(const IV *)(row + p.D + at);
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const unsigned bits = __builtin_bit_cast(unsigned, (float)xg[b][i]);
-        far = far > bits ? far : bits;
-      }
-      if (far > __builtin_bit_cast(unsigned, SILU_MIN)) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-          const float g = (float)xg[b][i];
-          if (g < SILU_MIN) v[b][i] = (float)xv[b][i] * (g / (1.0f + expf(-g)));
-        }
+        for (int i = 0; i < 8; i++)
+          if ((float)gt[i] < SILU_MIN) v[b][i] = (float)x[i] * silu_low((float)gt[i]);
       }
     }
     // columns 8 l32 + i: bits 0-2 in the lane, bits 3-7 across lanes
@@ -190,9 +202,13 @@ __global__ __launch_bounds__(256) void rot_q8_kernel(const char *__restrict__ in
     // |v rs| <= 127.5: adding 1.5 * 2^23 rounds to the nearest integer (half to even), whose two's complement is then
     // in the low bits. Not so where 1 / scale overflows (amax below 127 * 2^-128; the same for the whole row), and a NaN
     // of 32-bit rows may carry payload bits there (one of 16-bit rows has none so low): those are converted, so that a
-    // NaN has code 0.
-    if (IN_T == T_F32 || rs == INFINITY) store([](float y) { return (signed char)(int)rintf(y); });
-    else store([](float y) { return (signed char)__builtin_bit_cast(unsigned, y + 12582912.0f); });
+    // NaN has code 0. Rows of at most 8 blocks are too: one operation a value more, but no branch (16896 rows of 256
+    // columns 11.5 -> 10.8 us; 2048 columns 20 us either way, gated 38.7 -> 39.8).
+    const unsigned rsu = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(unsigned, rs));
+    if (IN_T == T_F32 || MAXB == 1 || __builtin_expect(rsu == __builtin_bit_cast(unsigned, INFINITY), 0))
+      store([](float y) { return (signed char)(int)rintf(y); });
+    else
+      store([](float y) { return (signed char)__builtin_bit_cast(unsigned, y + 12582912.0f); });
     if (threadIdx.x == 0) sa[m] = scale;
   }
 }
