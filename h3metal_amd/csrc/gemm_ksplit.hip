@@ -12,7 +12,7 @@
 // h8 weights stay int8 in LDS and are widened in registers (exact), so no widened copy of the weights is made.
 // Tiles are ordered down the rows first and each XCD takes a contiguous range, so that it reads its own columns of
 // W once and the (small) A from its L2.
-// Measured (us a call, 256 x 256 tiles -> here): 300 x 4096 x 4096 h8 99 -> 18.4, bf16 82 -> 18.8, q8 48 -> 14.2;
+// Measured (us a call, 256 x 256 tiles -> here): 300 x 4096 x 4096 h8 99 -> 18.8, bf16 82 -> 18.8, q8 48 -> 14.2;
 // 16 x 4096 x 4096 q8 44 -> 8.7; 128 x 2048 x 8192 q8 into the residual 89 -> 10.2.
 #include "gemm_common.h"
 
